@@ -50,7 +50,8 @@ struct ana_ctx {
            *d_step = nullptr;
   uint64_t* d_rng = nullptr;
   unsigned long long* d_amax = nullptr;  // [wb] greedy argmax keys
-  float *d_ss = nullptr, *d_pm = nullptr; // split attention scratch
+  float *d_ss = nullptr, *d_pm = nullptr; // split attention scratch, ss_rows rows
+  uint32_t ss_rows = 1;
   float* d_part = nullptr;           // fast attention's per-split partials
   size_t part_cap = 0;               // their floats
   float* SC = nullptr;               // scoring: the head's logits for up to sc_rows rows
@@ -358,8 +359,9 @@ extern "C" int ana_open(const char* path, const ana_opts* opts, ana_ctx** out) {
   if ((e = dalloc(&c->d_step, wb)) != hipSuccess) return bad(e);
   if ((e = dalloc(&c->d_out, wb * kOutSteps)) != hipSuccess) return bad(e);
   if ((e = dalloc(&c->d_amax, wb * kAmaxPerRow)) != hipSuccess) return bad(e);
-  if ((e = dalloc(&c->d_ss, wb * cf.heads * cf.ctx)) != hipSuccess) return bad(e);
-  if ((e = dalloc(&c->d_pm, wb * cf.heads * ((cf.ctx + kAttnTS - 1) / kAttnTS))) != hipSuccess) return bad(e);
+  c->ss_rows = std::max(c->wb, kAttnWideB);
+  if ((e = dalloc(&c->d_ss, (uint64_t)c->ss_rows * cf.heads * cf.ctx)) != hipSuccess) return bad(e);
+  if ((e = dalloc(&c->d_pm, (uint64_t)c->ss_rows * cf.heads * ((cf.ctx + kAttnTS - 1) / kAttnTS))) != hipSuccess) return bad(e);
   if ((e = dalloc(&c->QKV, (uint64_t)c->rows * 3 * d)) != hipSuccess) return bad(e);
   if ((e = dalloc(&c->Z, (uint64_t)c->rows * d)) != hipSuccess) return bad(e);
   if ((e = dalloc(&c->O, (uint64_t)c->rows * d)) != hipSuccess) return bad(e);
@@ -374,17 +376,19 @@ extern "C" int ana_open(const char* path, const ana_opts* opts, ana_ctx** out) {
       (e = dalloc(&c->d_tgt, c->rows)) != hipSuccess || (e = dalloc(&c->d_ce, c->rows)) != hipSuccess ||
       (e = dalloc(&c->d_stat, 3 * (uint64_t)c->max_seqs)) != hipSuccess)
     return bad(e);
-  // a prefill step's residual-row pairs (every mode)
-  if ((e = dalloc(&c->d_rcp, 2 * (uint64_t)c->rows)) != hipSuccess) return bad(e);
+  // a prefill step's residual-row pairs, chunks, and rows' sequences and
+  // positions (every mode)
+  if ((e = dalloc(&c->d_rcp, 2 * (uint64_t)c->rows)) != hipSuccess ||
+      (e = dalloc(&c->d_grun, c->seg_cap)) != hipSuccess || (e = dalloc(&c->d_rseq, c->rows)) != hipSuccess ||
+      (e = dalloc(&c->d_rpos, c->rows)) != hipSuccess)
+    return bad(e);
   if (c->mode != ANA_EXACT_FP32) {
     // the fast kernels' scratch: attention partials for every row of a step,
     // the GLA scan's regions and tables
     c->part_cap = attn_fast_part_floats(c->rows, cf.heads, cf.ctx, hd);
     if ((e = dalloc(&c->d_part, c->part_cap)) != hipSuccess ||
         (e = dalloc(&c->d_gla, gla_scan_floats(c->rows, c->gsub_cap, c->seg_cap, d, cf.heads))) != hipSuccess ||
-        (e = dalloc(&c->d_gtab, c->gsub_cap)) != hipSuccess || (e = dalloc(&c->d_grun, c->seg_cap)) != hipSuccess ||
-        (e = dalloc(&c->d_atab, c->atab_cap)) != hipSuccess ||
-        (e = dalloc(&c->d_rseq, c->rows)) != hipSuccess || (e = dalloc(&c->d_rpos, c->rows)) != hipSuccess)
+        (e = dalloc(&c->d_gtab, c->gsub_cap)) != hipSuccess || (e = dalloc(&c->d_atab, c->atab_cap)) != hipSuccess)
       return bad(e);
     c->gla = gla_scan_carve(c->d_gla, c->rows, c->gsub_cap, c->seg_cap, d, cf.heads);
   }
@@ -803,31 +807,33 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
   c->nx_of = nullptr;
   c->oh_ok = false;
   const bool bf_ops = c->d_oh && chunk && B >= 128 && B <= c->rows && d % 64 == 0;
-  // a fast mode's prefill step: the GLA scan's sub-chunk table and each row's
-  // sequence and position, uploaded once for every layer
+  // a prefill step: its chunks, the GLA scan's sub-chunk table (the fast
+  // modes) and each row's sequence and position, uploaded once for every
+  // layer
   uint32_t nsub = 0;
   bool fresh_all = true, gla_run = true;
-  if (chunk && fast_mode(c)) {
+  if (chunk) {
     if (segs->size() > c->seg_cap) return fail(c, ANA_EINVAL, "prefill step of %zu chunks (at most %u)", segs->size(), c->seg_cap);
     c->h_gtab.clear();
     c->h_grun.clear();
     c->h_atab.clear();
     // attention tile rows: 128 on the bf16 flash kernel, else 64
     const uint32_t fq = attn_flash_tile_rows(c->mode == ANA_BF16, d / cf.heads);
+    const bool fast = fast_mode(c);
     c->h_rseq.resize(B);
     c->h_rpos.resize(B);
     for (uint32_t si = 0; si < segs->size(); si++) {
       const Seg& sg = (*segs)[si];
       const uint32_t ns = (sg.T + kGlaSub - 1) / kGlaSub;
-      for (uint32_t j = 0; j < ns; j++)
+      for (uint32_t j = 0; fast && j < ns; j++)
         c->h_gtab.push_back(GlaSub{sg.row0 + j * kGlaSub, std::min(kGlaSub, sg.T - j * kGlaSub), j, ns, sg.seq, si, 0, 0});
       c->h_grun.push_back(GlaRun{sg.row0, sg.T, sg.seq, 0});
-      if (sg.T > kGlaRunMaxT) gla_run = false;
+      if (fast && sg.T > kGlaRunMaxT) gla_run = false;
       for (uint32_t t = 0; t < sg.T; t++) {
         c->h_rseq[sg.row0 + t] = sg.seq;
         c->h_rpos[sg.row0 + t] = sg.pos0 + t;
       }
-      for (uint32_t t = 0; t < sg.T; t += fq)
+      for (uint32_t t = 0; fast && t < sg.T; t += fq)
         c->h_atab.push_back(AttnTile{sg.seq, sg.pos0 + t, sg.row0 + t, std::min(fq, sg.T - t)});
       const uint64_t last = (uint64_t)sg.pos0 + sg.T - 1;
       if (last >= cf.ctx) fresh_all = false;
@@ -875,12 +881,8 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
         HIPCHK(c, launch_gla_scan(c->QKV, c->Z, cf.rglru ? W + b.lam : nullptr, sref(c, l), c->O, c->gla,
                                   c->d_gtab, nsub, d, cf.heads, cf.rglru, c->st));
     } else if (b.gla) {
-      for (const Seg& sg : *segs) {
-        float* S = c->state + (uint64_t)sg.seq * c->seq_stride + c->layer_off[l];
-        HIPCHK(c, launch_gla_chunk(c->QKV + (size_t)sg.row0 * 3 * d, c->Z + (size_t)sg.row0 * d,
-                                   cf.rglru ? W + b.lam : nullptr, S, c->O + (size_t)sg.row0 * d, d,
-                                   cf.heads, cf.rglru, sg.T, c->st));
-      }
+      HIPCHK(c, launch_gla_serial(c->QKV, c->Z, cf.rglru ? W + b.lam : nullptr, sref(c, l), c->O, c->d_grun,
+                                  (uint32_t)c->h_grun.size(), d, cf.heads, cf.rglru, c->st));
     } else {
       AttnArgs a{};
       a.gq = cf.qk ? W + b.gq : nullptr;
@@ -888,7 +890,7 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
       a.sink = cf.sinks ? W + b.sink : nullptr;
       a.KV = sref(c, l);
       a.d = d; a.heads = cf.heads; a.ctx = cf.ctx;
-      a.ss = c->d_ss; a.pm = c->d_pm; a.ss_rows = c->wb;
+      a.ss = c->d_ss; a.pm = c->d_pm; a.ss_rows = c->ss_rows;
       a.part_cap = c->part_cap;
       if (!chunk) {
         // each sequence's write, then its attention (dd.sm.write, dd.sm.attend)
@@ -911,6 +913,12 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
         a.Oh = bf_ops ? c->d_oh : nullptr;
         HIPCHK(c, launch_attn_flash(a, c->d_atab, (uint32_t)c->h_atab.size(), c->mode == ANA_BF16, c->st));
         c->oh_ok = bf_ops;
+      } else if (fresh_all) {
+        // the exact mode: every row's write, then every row's attention
+        // (dd.sm.writes, then dd.sm.rows, for every chunk)
+        a.QKV = c->QKV; a.O = c->O; a.B = B; a.seq = c->d_rseq; a.pos = c->d_rpos; a.write_kv = 0;
+        HIPCHK(c, launch_kv_write(a, c->st));
+        HIPCHK(c, launch_attn(a, c->st));
       } else {
         for (const Seg& sg : *segs) {
           const bool fresh = (uint64_t)sg.pos0 + sg.T <= cf.ctx;

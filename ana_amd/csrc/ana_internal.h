@@ -160,10 +160,19 @@ hipError_t launch_bswap(uint32_t* w, uint64_t n, hipStream_t st);
 hipError_t launch_gla_step(const float* QKV, const float* Z, const float* lam, StateRef S,
                            const uint32_t* seq, float* O, uint32_t d, uint32_t heads,
                            uint32_t rglru, uint32_t B, hipStream_t st);
-// GLA over T tokens of one sequence, token after token (S kept on chip).
-hipError_t launch_gla_chunk(const float* QKV, const float* Z, const float* lam, float* S,
-                            float* O, uint32_t d, uint32_t heads, uint32_t rglru, uint32_t T,
-                            hipStream_t st);
+// One chunk of a prefill step: T tokens of the sequence in state slot seq,
+// from workspace row `row`.
+struct GlaRun {
+  uint32_t row;   // first workspace row
+  uint32_t T;     // tokens
+  uint32_t seq;   // state slot
+  uint32_t pad;
+};
+// GLA over a prefill step's chunks (at least one token each), token after
+// token, S kept on chip: every chunk in one launch.
+hipError_t launch_gla_serial(const float* QKV, const float* Z, const float* lam, StateRef S, float* O,
+                             const GlaRun* runs, uint32_t nrun, uint32_t d, uint32_t heads, uint32_t rglru,
+                             hipStream_t st);
 
 // Softmax attention over the ring for B (seq, pos) rows. write_kv: each
 // row writes its own k (qk-normed) and v into its slot first (the decode
@@ -194,6 +203,10 @@ struct AttnArgs {
 constexpr uint32_t kFastTS = 64;
 // slots per workgroup in the split attention's score pass
 constexpr uint32_t kAttnTS = 128;
+// from kAttnWideB rows on, one workgroup per (head, row) (k_attn) keeps
+// every CU busy, and the split kernels would dispatch ctx / kAttnTS score
+// blocks per (head, row) whatever the row's position
+constexpr uint32_t kAttnWideB = 8;
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st);
 // each row's k (qk-normed when gk) and v into slot pos mod ctx (dd.sm.write)
 hipError_t launch_kv_write(const AttnArgs& a, hipStream_t st);
@@ -307,16 +320,10 @@ struct GlaScratch {
   float *Qt, *Dj, *Uj, *S0;
   uint32_t rows_cap, nsub_cap, nseg_cap;  // what the regions were carved for
 };
-// One chunk of a prefill step for k_gla_run: one workgroup per (head,
-// chunk) walks its sub-chunks in order, the state in LDS. Chunks of at most
+// k_gla_run: one workgroup per (head, chunk) walks the chunk's sub-chunks
+// in order, the state in LDS. Chunks of at most
 // kGlaRunMaxT tokens take it (a few sequential sub-chunks, and a tenth of
 // the scan's traffic); longer ones the scan.
-struct GlaRun {
-  uint32_t row;   // first workspace row
-  uint32_t T;     // tokens
-  uint32_t seq;   // state slot
-  uint32_t pad;
-};
 constexpr uint32_t kGlaRunMaxT = 8 * kGlaSub;
 // (rows: the workspace rows QKV and Z hold)
 // (Oh: the outputs in bf16 only, for a bf16 Wo operand)

@@ -575,77 +575,222 @@ hipError_t launch_bswap(uint32_t* w, uint64_t n, hipStream_t st) {
 // ------------------------------------------------------------------ GLA
 
 // dd.gla's per-token part (bend/Dense/Decode.bend:252-266, 275-290) for one
-// head: L2 norms (M.l2), the gate (dd.gate: RG-LRU or sigmoid), the state
-// update S' = al*S + kh*v and the readout o = qh^T S' (no 1/sqrt(hd)).
-// nT tokens run in order, S staying in LDS between them.
+// (head, sequence) of a decode step whose hd is not 64: L2 norms (M.l2), the
+// gate (dd.gate: RG-LRU or sigmoid), the state update S' = al*S + kh*v and
+// the readout o = qh^T S' (no 1/sqrt(hd)).
 template <int HD>
 __global__ __launch_bounds__(256) void k_gla(const float* __restrict__ QKV,
                                               const float* __restrict__ Z,
                                               const float* __restrict__ lam, StateRef S,
-                                              const uint32_t* __restrict__ seq, uint32_t seq0,
-                                              float* __restrict__ O, uint32_t d, uint32_t rglru,
-                                              uint32_t nT) {
+                                              const uint32_t* __restrict__ seq,
+                                              float* __restrict__ O, uint32_t d, uint32_t rglru) {
   constexpr int SP = HD + 1;
   constexpr int NE = (HD * HD + 255) / 256;
   __shared__ float q[HD], k[HD], v[HD], z[HD], al[HD], kh[HD], qh[HD], sq[2];
   __shared__ float Sl[HD * SP];
   const uint32_t h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
-  const uint32_t sl = seq ? seq[b] : seq0;
-  float* Sg = S.base + (size_t)sl * S.seq_stride + S.layer_off + (size_t)h * HD * HD;
+  float* Sg = S.base + (size_t)seq[b] * S.seq_stride + S.layer_off + (size_t)h * HD * HD;
 #pragma unroll
   for (int j = 0; j < NE; j++) {
     const uint32_t e = tid + 256 * j;
     if (e < HD * HD) Sl[(e / HD) * SP + (e % HD)] = Sg[e];
   }
-  for (uint32_t t = 0; t < nT; t++) {
-    const uint32_t row = seq ? b : t;   // batch row (step) or token row (chunk)
-    const float* x = QKV + (size_t)row * 3 * d;
-    __syncthreads();
-    if (tid < HD) {
-      q[tid] = x[h * HD + tid];
-      k[tid] = x[d + h * HD + tid];
-      v[tid] = x[2 * d + h * HD + tid];
-      z[tid] = Z[(size_t)row * d + h * HD + tid];
-    }
-    __syncthreads();
-    if (tid == 0) sq[0] = chain_sumsq_lds(0.0f, q, HD);
-    else if (tid == 64) sq[1] = chain_sumsq_lds(0.0f, k, HD);
-    __syncthreads();
-    if (tid < HD) {
-      qh[tid] = q[tid] / csqrt(1.0e-6f + sq[0]);
-      const float kn = k[tid] / csqrt(1.0e-6f + sq[1]);
-      if (rglru) {
-        const float la = ex_rglru_log_gate(z[tid], lam[h * HD + tid]);
-        kh[tid] = kn * ex_rglru_write_scale(la);
-        al[tid] = dexp(la);
-      } else {
-        al[tid] = ex_sigmoid(z[tid]);
-        kh[tid] = kn;
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < NE; j++) {
-      const uint32_t e = tid + 256 * j;
-      if (e < HD * HD) {
-        const uint32_t ia = e / HD, ib = e % HD;
-        float* p = &Sl[ia * SP + ib];
-        *p = (al[ia] * *p) + (kh[ia] * v[ib]);
-      }
-    }
-    __syncthreads();
-    if (tid < HD) {
-      float acc = 0.0f;
-#pragma unroll
-      for (int i = 0; i < HD; i++) acc = acc + qh[i] * Sl[i * SP + tid];
-      O[(size_t)row * d + h * HD + tid] = acc;
+  const float* x = QKV + (size_t)b * 3 * d;
+  if (tid < HD) {
+    q[tid] = x[h * HD + tid];
+    k[tid] = x[d + h * HD + tid];
+    v[tid] = x[2 * d + h * HD + tid];
+    z[tid] = Z[(size_t)b * d + h * HD + tid];
+  }
+  __syncthreads();
+  if (tid == 0) sq[0] = chain_sumsq_lds(0.0f, q, HD);
+  else if (tid == 64) sq[1] = chain_sumsq_lds(0.0f, k, HD);
+  __syncthreads();
+  if (tid < HD) {
+    qh[tid] = q[tid] / csqrt(1.0e-6f + sq[0]);
+    const float kn = k[tid] / csqrt(1.0e-6f + sq[1]);
+    if (rglru) {
+      const float la = ex_rglru_log_gate(z[tid], lam[h * HD + tid]);
+      kh[tid] = kn * ex_rglru_write_scale(la);
+      al[tid] = dexp(la);
+    } else {
+      al[tid] = ex_sigmoid(z[tid]);
+      kh[tid] = kn;
     }
   }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < NE; j++) {
     const uint32_t e = tid + 256 * j;
-    if (e < HD * HD) Sg[e] = Sl[(e / HD) * SP + (e % HD)];
+    if (e < HD * HD) {
+      const uint32_t ia = e / HD, ib = e % HD;
+      float* p = &Sl[ia * SP + ib];
+      const float s1 = (al[ia] * *p) + (kh[ia] * v[ib]);
+      *p = s1;
+      Sg[e] = s1;
+    }
+  }
+  __syncthreads();
+  if (tid < HD) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int i = 0; i < HD; i++) acc = acc + qh[i] * Sl[i * SP + tid];
+    O[(size_t)b * d + h * HD + tid] = acc;
+  }
+}
+
+// dd.gla over a prefill step's chunks, token after token, one workgroup per
+// (head, chunk): every chunk of the step in one launch. What a token's
+// update needs besides the state (qh, kh, al) depends on no other token, so
+// three waves form it for kSerialT tokens at a time (the norms' chains, a
+// lane each; the gates through double) while the fourth runs the tokens
+// before them: lane b keeps column b of the head's state in registers and
+// takes k_gla's operations in k_gla's order, S' = (al_a S) + (kh_a v_b) and
+// o_b = ((0 + qh_0 S'_0b) + qh_1 S'_1b) + ..., its rows' al, kh and qh read
+// from LDS eight at a time, a group ahead of the one it works on.
+// The serial wave bounds it: 5 operations a row, 64 rows a token, 4 cycles
+// an operation is 0.53 us a token at 2.4 GHz. One workgroup per head a
+// launch, a launch a chunk, every wave meeting at five barriers a token
+// (which this replaced) took 215 us for 64 tokens of one sequence, so 1.7 ms
+// for eight; this takes 58 us for the eight together (115M, hd 64).
+constexpr int kSerialT = 12;
+template <int HD>
+__global__ __launch_bounds__(256) void k_gla_serial(const float* __restrict__ QKV, const float* __restrict__ Z,
+                                                     const float* __restrict__ lam, StateRef S,
+                                                     float* __restrict__ O, const GlaRun* __restrict__ runs,
+                                                     uint32_t d, uint32_t rglru) {
+  constexpr int NP = kSerialT / 3, RP = HD + 4, NG = HD / 8;   // tokens a wave prepares; raw row pitch; row groups
+  static_assert(kSerialT % 3 == 0 && 2 * NP <= 64 && HD % 16 == 0, "token and row groups");
+  struct Tok { float al[HD], kh[HD], qh[HD], v[HD]; };
+  __shared__ __align__(16) Tok tk[2][kSerialT];
+  __shared__ __align__(16) float raw[3][2 * NP][RP];           // a wave's q and k rows, in turn
+  const uint32_t h = blockIdx.x, lane = threadIdx.x & 63;
+  const GlaRun run = runs[blockIdx.y];
+  // the serial wave: another one for the workgroups that a CU holds at once
+  // (ids 256 apart), so they do not meet on one SIMD
+  const uint32_t sw = ((blockIdx.x + blockIdx.y * gridDim.x) >> 8) & 3;
+  const uint32_t wv = (threadIdx.x >> 6) ^ sw;                 // 0: the serial wave
+  const uint32_t T = run.T, nb = (T + kSerialT - 1) / kSerialT;
+  const bool on = lane < (uint32_t)HD;
+  const uint32_t col = h * HD + (on ? lane : 0);
+  const float lv = rglru ? lam[col] : 0.0f;
+  auto prep = [&](uint32_t j) {
+    const uint32_t w = wv - 1;
+    Tok* out = tk[j & 1];
+    float q[NP], k[NP], v[NP], z[NP];
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const uint32_t t = min(j * kSerialT + 3 * i + w, T - 1);
+      const float* x = QKV + (size_t)(run.row + t) * 3 * d;
+      q[i] = x[col];
+      k[i] = x[d + col];
+      v[i] = x[2 * d + col];
+      z[i] = Z[(size_t)(run.row + t) * d + col];
+    }
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < NP; i++) {
+        raw[w][2 * i][lane] = q[i];
+        raw[w][2 * i + 1][lane] = k[i];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const float sq = chain_sumsq_lds(0.0f, raw[w][lane % (2 * NP)], HD);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < NP; i++) {
+      const float s0 = __shfl(sq, 2 * i, 64), s1 = __shfl(sq, 2 * i + 1, 64);
+      const float kn = k[i] / csqrt(1.0e-6f + s1);
+      float alv, khv;
+      if (rglru) {
+        const float la = ex_rglru_log_gate(z[i], lv);
+        khv = kn * ex_rglru_write_scale(la);
+        alv = dexp(la);
+      } else {
+        alv = ex_sigmoid(z[i]);
+        khv = kn;
+      }
+      if (on) {
+        Tok& t = out[3 * i + w];
+        t.al[lane] = alv;
+        t.kh[lane] = khv;
+        t.qh[lane] = q[i] / csqrt(1.0e-6f + s0);
+        t.v[lane] = v[i];
+      }
+    }
+  };
+  float s[HD];
+  float* Sg = S.base + (size_t)run.seq * S.seq_stride + S.layer_off + (size_t)h * HD * HD + (on ? lane : 0);
+  if (wv == 0) {
+#pragma unroll
+    for (int a = 0; a < HD; a++) s[a] = Sg[a * HD];
+  }
+  struct Rows { float4 al[2], kh[2], qh[2]; };
+  auto serial = [&](uint32_t j) {
+    const Tok* in = tk[j & 1];
+    const uint32_t n = min((uint32_t)kSerialT, T - j * kSerialT);
+    auto load = [&](Rows& r, uint32_t t, int g) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        r.al[u] = *reinterpret_cast<const float4*>(&in[t].al[8 * g + 4 * u]);
+        r.kh[u] = *reinterpret_cast<const float4*>(&in[t].kh[8 * g + 4 * u]);
+        r.qh[u] = *reinterpret_cast<const float4*>(&in[t].qh[8 * g + 4 * u]);
+      }
+    };
+    float acc = 0.0f, vv = in[0].v[on ? lane : 0];
+    auto rows8 = [&](const Rows& r, int g) {
+      auto row = [&](float al, float kh, float qh, int a) {
+        s[a] = (al * s[a]) + (kh * vv);
+        acc = acc + qh * s[a];
+      };
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        row(r.al[u].x, r.kh[u].x, r.qh[u].x, 8 * g + 4 * u);
+        row(r.al[u].y, r.kh[u].y, r.qh[u].y, 8 * g + 4 * u + 1);
+        row(r.al[u].z, r.kh[u].z, r.qh[u].z, 8 * g + 4 * u + 2);
+        row(r.al[u].w, r.kh[u].w, r.qh[u].w, 8 * g + 4 * u + 3);
+      }
+    };
+    // (nothing moved across: the reads of a group stay ahead of the group
+    // before it)
+    auto keep = [&]() { __builtin_amdgcn_sched_barrier(0); };
+    Rows ra, rb;
+    load(ra, 0, 0);
+    for (uint32_t t = 0; t < n; t++) {
+      acc = 0.0f;
+      const uint32_t tn = t + 1 < n ? t + 1 : t;
+      float vn = vv;
+#pragma unroll
+      for (int g = 0; g < NG; g += 2) {
+        load(rb, t, g + 1);
+        keep();
+        rows8(ra, g);
+        keep();
+        if (g + 2 < NG) {
+          load(ra, t, g + 2);
+        } else {
+          vn = in[tn].v[on ? lane : 0];
+          load(ra, tn, 0);
+        }
+        keep();
+        rows8(rb, g + 1);
+        keep();
+      }
+      if (on) O[(size_t)(run.row + j * kSerialT + t) * d + col] = acc;
+      vv = vn;
+    }
+  };
+  if (wv != 0) prep(0);
+  for (uint32_t j = 0; j < nb; j++) {
+    __syncthreads();
+    if (wv == 0) serial(j);
+    else if (j + 1 < nb) prep(j + 1);
+  }
+  if (wv == 0 && on) {
+#pragma unroll
+    for (int a = 0; a < HD; a++) Sg[a * HD] = s[a];
   }
 }
 
@@ -717,17 +862,17 @@ hipError_t launch_gla_step(const float* QKV, const float* Z, const float* lam, S
     hipLaunchKernelGGL(k_gla_w, dim3(heads, B), dim3(64), 0, st, QKV, Z, lam, S, seq, O, d, rglru);
     return hipGetLastError();
   }
-#define L_(H) hipLaunchKernelGGL(k_gla<H>, dim3(heads, B), dim3(256), 0, st, QKV, Z, lam, S, seq, 0u, O, d, rglru, 1u)
+#define L_(H) hipLaunchKernelGGL(k_gla<H>, dim3(heads, B), dim3(256), 0, st, QKV, Z, lam, S, seq, O, d, rglru)
   ANA_HD_DISPATCH(d / heads, L_)
 #undef L_
   return hipGetLastError();
 }
 
-hipError_t launch_gla_chunk(const float* QKV, const float* Z, const float* lam, float* Sbase,
-                            float* O, uint32_t d, uint32_t heads, uint32_t rglru, uint32_t T,
-                            hipStream_t st) {
-  StateRef S{Sbase, 0, 0};
-#define L_(H) hipLaunchKernelGGL(k_gla<H>, dim3(heads, 1), dim3(256), 0, st, QKV, Z, lam, S, (const uint32_t*)nullptr, 0u, O, d, rglru, T)
+hipError_t launch_gla_serial(const float* QKV, const float* Z, const float* lam, StateRef S, float* O,
+                             const GlaRun* runs, uint32_t nrun, uint32_t d, uint32_t heads, uint32_t rglru,
+                             hipStream_t st) {
+  if (nrun == 0) return hipErrorInvalidValue;
+#define L_(H) hipLaunchKernelGGL(k_gla_serial<H>, dim3(heads, nrun), dim3(256), 0, st, QKV, Z, lam, S, O, runs, d, rglru)
   ANA_HD_DISPATCH(d / heads, L_)
 #undef L_
   return hipGetLastError();
@@ -1019,11 +1164,6 @@ __global__ __launch_bounds__(256) void k_attn_out(AttnArgs a) {
   __syncthreads();
   if (tid < ATTN_CG) a.O[(size_t)b * d + h * HD + c0 + tid] = (1.0f / red[0]) * oi;
 }
-
-// From kAttnWideB rows on, one workgroup per (head, row) (k_attn) keeps
-// every CU busy, and the split kernels would dispatch ctx / kAttnTS score
-// blocks per (head, row) whatever the row's position.
-constexpr uint32_t kAttnWideB = 8;
 
 hipError_t launch_attn(const AttnArgs& a, hipStream_t st) {
   const uint32_t hd = a.d / a.heads;
