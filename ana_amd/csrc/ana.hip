@@ -79,6 +79,13 @@ struct ana_ctx {
   // bf16 in ANA_BF16; the norm gains folded in), found by the product's first
   // weight row; the entry keeps the segment shape and gains it was packed for
   void* PK = nullptr;
+  // ANA_FAST_FP32 prefill (use_x3): every product's weights in three bf16
+  // parts, found by the product's first weight row, a product's activations
+  // in parts, and gate|up's hidden rows (down's input, when hh3)
+  bool use_x3 = false, hh3 = false;
+  char* W3 = nullptr;
+  void *d_a3 = nullptr, *d_h3 = nullptr;
+  std::unordered_map<const float*, uint64_t> w3;
   unsigned long long* d_hpc = nullptr;  // the fused head and sampler's arrival counters
   uint32_t* d_hpctl = nullptr;          // and its ran-out flag
   struct PkEnt {
@@ -256,7 +263,7 @@ static void release(ana_ctx* c) {
   void* ps[] = {c->d_play, c->d_ctl, c->d_trace, c->W, c->Wh, c->Wp, c->d_part, c->d_gla, c->state, c->xs, c->X, c->XA, c->XN, c->QKV, c->Z, c->O, c->HH, c->LG,
                 c->d_seq, c->d_pos, c->d_tok, c->d_pick, c->d_out, c->d_step, c->d_rng, c->d_amax,
                 c->d_ss, c->d_pm, c->d_gtab, c->d_grun, c->d_atab, c->d_rseq, c->d_rpos, c->SC, c->d_tgt, c->d_ce, c->d_stat, c->d_rcp,
-                c->d_sah, c->d_hh, c->d_rsc, c->PK, c->d_hpc, c->d_hpctl, c->d_oh, c->d_nxh, c->d_ssp};
+                c->d_sah, c->d_hh, c->d_rsc, c->PK, c->W3, c->d_a3, c->d_h3, c->d_hpc, c->d_hpctl, c->d_oh, c->d_nxh, c->d_ssp};
   for (void* p : ps)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
@@ -291,6 +298,7 @@ extern "C" void ana_rng_seeded(uint64_t seed, uint64_t r[4]) {
 }
 
 static hipError_t pack_weights(ana_ctx* c);
+static hipError_t pack_parts(ana_ctx* c);
 static hipError_t persist_setup(ana_ctx* c);
 static void resolve_scratch(int device);
 
@@ -405,6 +413,7 @@ extern "C" int ana_open(const char* path, const ana_opts* opts, ana_ctx** out) {
   if ((e = launch_bswap(reinterpret_cast<uint32_t*>(c->W), c->P, c->st)) != hipSuccess) return bad(e);
   if (c->Wh && (e = launch_to_bf16(c->W, c->Wh, c->P, c->st)) != hipSuccess) return bad(e);
   if (c->mode != ANA_EXACT_FP32 && (e = pack_weights(c)) != hipSuccess) return bad(e);
+  if (c->mode == ANA_FAST_FP32 && (e = pack_parts(c)) != hipSuccess) return bad(e);
   if (c->mode != ANA_EXACT_FP32) {
     // the fused head and sampler's counters (one per 32-row block, only
     // ever added to) and flag start at zero
@@ -515,6 +524,9 @@ static bool reads_bf16(const ana_ctx* c, const GemvArgs& g) {
   return !(o >= c->fp32_lo && o < c->fp32_hi);
 }
 
+static const uint32_t kBigB = 128;   // prefill steps of this many rows or more take the big tiles
+static hipError_t launch_x3(ana_ctx* c, const GemvArgs& g, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+
 // next_gain: the norm gain of the product that reads this one's outputs
 // next (a prefill step's residual products), for a producer-side bf16 copy
 static hipError_t gemv_timed(ana_ctx* c, const GemvArgs& g0, uint32_t kind, bool chunk = false,
@@ -532,16 +544,20 @@ static hipError_t gemv_timed(ana_ctx* c, const GemvArgs& g0, uint32_t kind, bool
   // the hidden rows exist only in bf16 after a gate|up that wrote d_hh, so
   // down must take the path that reads them there
   const bool hh_only = (g0.X == c->HH && hh_was) || oh_here;   // (or O, when the mix left it in bf16 only)
+  if (c->use_x3 && chunk && g0.B >= kBigB) {
+    ProfScope ps(c, kind, gemv_bytes(g0), true);
+    return launch_x3(c, g0, ps.start(), ps.stop());
+  }
   const bool pk_ok = gemm_pk_fits(g0) || (kind == ANA_K_HEAD && head_pw_fits(g0));
   const ana_ctx::PkEnt* pe =
-      fast_mode(c) && !small && g0.B < (chunk ? 128u : kPwMaxB) && pk_ok ? find_pk(c, g0) : nullptr;
+      fast_mode(c) && !small && g0.B < (chunk ? kBigB : kPwMaxB) && pk_ok ? find_pk(c, g0) : nullptr;
   // the head of a decode step of kPwMaxB rows or more takes the prefill
   // products too (greedy picks then read the stored logits)
   if (pe || (fast_mode(c) && (small ? !chunk : (chunk || kind != ANA_K_HEAD || g0.B >= kPwMaxB)))) {
     GemvArgs g = g0;
     // prefill steps on the big tiles read every block's weights in bf16
     // (decode keeps the first block in fp32)
-    const bool bf = reads_bf16(c, g) || (c->Wh && chunk && g.B >= 128);
+    const bool bf = reads_bf16(c, g) || (c->Wh && chunk && g.B >= kBigB);
     if (bf) {
       g.Wh0 = c->Wh + (g.seg[0].W - c->W);
       g.Wh1 = g.nseg > 1 ? c->Wh + (g.seg[1].W - c->W) : nullptr;
@@ -555,7 +571,7 @@ static hipError_t gemv_timed(ana_ctx* c, const GemvArgs& g0, uint32_t kind, bool
       return launch_head_pw(g, static_cast<const char*>(c->PK) + pe->off, pe->bf, c->st, ps.start(), ps.stop());
     if (pe)
       return launch_gemm_pk(g, static_cast<const char*>(c->PK) + pe->off, pe->bf, c->st, ps.start(), ps.stop());
-    if (g.B >= 128 && c->d_sah && bf && g.K % 64 == 0 && g.B <= c->rows) {
+    if (g.B >= kBigB && c->d_sah && bf && g.K % 64 == 0 && g.B <= c->rows) {
       // gate|up leaves its outputs in bf16 only, and down reads them there
       // instead of splitting them again
       if (g.mode == GM_SILU && c->d_hh && gemm_wide_takes(g)) g.Yh = c->d_hh;
@@ -588,7 +604,7 @@ static hipError_t gemv_timed(ana_ctx* c, const GemvArgs& g0, uint32_t kind, bool
       return e;
     }
     if (hh_only) return hipErrorInvalidValue;
-    if (g.B >= 128) return launch_gemm_big(g, c->st, ps.start(), ps.stop());
+    if (g.B >= kBigB) return launch_gemm_big(g, c->st, ps.start(), ps.stop());
     return launch_gemm_mfma(g, c->st, ps.start(), ps.stop());
   }
   if (hh_only) return hipErrorInvalidValue;
@@ -774,6 +790,56 @@ static hipError_t pack_weights(ana_ctx* c) {
   return hipSuccess;
 }
 
+// ANA_FAST_FP32: every product's weights in three bf16 parts, and the room
+// for a prefill step's activations in parts, where every product of the
+// model fits the split tiles and a prefill step can have the rows for them
+static hipError_t pack_parts(ana_ctx* c) {
+  const ana_config& cf = c->cfg;
+  if (c->rows < kBigB) return hipSuccess;
+  std::vector<GemvArgs> all;
+  for (uint32_t l = 0; l < cf.layers; l++) {
+    GemvArgs p[4];
+    layer_products(c, l, p);
+    for (const GemvArgs& g : p) {
+      if (!x3_fits(g)) return hipSuccess;
+      all.push_back(g);
+    }
+  }
+  GemvArgs h = gemv1(c->X, cf.d, cf.d, c->W, cf.vocab, c->SC, cf.vocab, 0);
+  h.ng = c->W + c->fin;
+  if (x3_fits(h)) all.push_back(h);
+  uint64_t total = 0;
+  for (const GemvArgs& g : all) {
+    c->w3[g.seg[0].W] = total;
+    total += x3_weight_bytes(g);
+  }
+  hipError_t e;
+  if ((e = dalloc(&c->W3, total)) != hipSuccess ||
+      (e = hipMalloc(&c->d_a3, x3_bytes(c->rows, cf.d))) != hipSuccess ||
+      (e = hipMalloc(&c->d_h3, x3_bytes(c->rows, cf.f))) != hipSuccess || (e = dalloc(&c->d_rsc, c->rows)) != hipSuccess)
+    return e;
+  for (const GemvArgs& g : all)
+    if ((e = launch_pack3(g, c->W3 + c->w3[g.seg[0].W], c->st)) != hipSuccess) return e;
+  c->use_x3 = true;
+  return hipSuccess;
+}
+
+// a prefill product on the split tiles: its input in parts first, unless
+// gate|up left it so
+static hipError_t launch_x3(ana_ctx* c, const GemvArgs& g, hipEvent_t e0, hipEvent_t e1) {
+  const auto it = c->w3.find(g.seg[0].W);
+  if (it == c->w3.end() || g.B > c->rows) return hipErrorInvalidValue;
+  if (e0) (void)hipEventRecord(e0, c->st);
+  const bool hidden = g.X == c->HH && c->hh3;
+  hipError_t e = hipSuccess;
+  if (!hidden) e = launch_split3(g.X, g.ldx, g.K, g.B, c->d_a3, g.ng ? c->d_rsc : nullptr, c->st);
+  if (e == hipSuccess)
+    e = launch_gemm_x3(g, hidden ? c->d_h3 : c->d_a3, c->W3 + it->second, c->d_rsc, c->d_h3, c->st);
+  c->hh3 = g.mode == GM_SILU && e == hipSuccess;
+  if (e1) (void)hipEventRecord(e1, c->st);
+  return e;
+}
+
 // RMSNorm(X; g) then the product: inside the product for small batches,
 // else a norm kernel into XN first
 static int norm_gemv(ana_ctx* c, const float* X, const float* g, GemvArgs a, uint32_t kind,
@@ -806,7 +872,7 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
   // write Wo's operand in bf16 and the residual products the next norm's
   c->nx_of = nullptr;
   c->oh_ok = false;
-  const bool bf_ops = c->d_oh && chunk && B >= 128 && B <= c->rows && d % 64 == 0;
+  const bool bf_ops = c->d_oh && chunk && B >= kBigB && B <= c->rows && d % 64 == 0;
   // a prefill step: its chunks, the GLA scan's sub-chunk table (the fast
   // modes) and each row's sequence and position, uploaded once for every
   // layer
@@ -1047,7 +1113,9 @@ static int score_head(ana_ctx* c, uint32_t r0, uint32_t g) {
     // ANA_BF16 at 128 rows or more: the bf16 matrix-core tiles, as the
     // layer products of a prefill step (activations rounded to bf16 with
     // the final norm's gain, as the decode head rounds them)
-    if (c->Wh && c->d_sah && g >= 128 && cf.d % 64 == 0)
+    if (c->use_x3 && g >= kBigB && c->w3.count(h.seg[0].W))
+      HIPCHK(c, launch_x3(c, h));
+    else if (c->Wh && c->d_sah && g >= kBigB && cf.d % 64 == 0)
       HIPCHK(c, launch_gemm_dl(h, c->d_sah, c->d_rsc, c->rows, c->st));
     else
       HIPCHK(c, launch_gemm_big(h, c->st));

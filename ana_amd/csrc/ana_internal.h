@@ -375,6 +375,19 @@ hipError_t launch_head_pw(const GemvArgs& a, const void* pk, int bf, hipStream_t
 // the same for 128 rows or more, 128 x 128 tiles
 hipError_t launch_gemm_big(const GemvArgs& a, hipStream_t st, hipEvent_t e0 = nullptr,
                            hipEvent_t e1 = nullptr);
+// ANA_FAST_FP32 products on the bf16 matrix cores, operands in three bf16
+// parts (gemm_split.hip): whether a product's shape fits (K a multiple of
+// 32, whole 16-row weight tiles), the bytes of an operand of `rows` x K in
+// parts, the weights' packing (norm gains folded in), the activations' (and
+// with rsc the rows' norm scales), and the product itself (A from
+// launch_split3, or the hidden rows H that a SiLU product leaves in parts
+// instead of writing its outputs; rsc when g.ng)
+bool x3_fits(const GemvArgs& g);
+uint64_t x3_bytes(uint32_t rows, uint32_t K);
+uint64_t x3_weight_bytes(const GemvArgs& g);
+hipError_t launch_pack3(const GemvArgs& g, void* dst, hipStream_t st);
+hipError_t launch_split3(const float* X, uint32_t ldx, uint32_t K, uint32_t B, void* dst, float* rsc, hipStream_t st);
+hipError_t launch_gemm_x3(const GemvArgs& g, const void* A, const void* W, const float* rsc, void* H, hipStream_t st);
 // ANA_BF16 at 128 rows or more: the activations (times the norm's gain)
 // rounded to bf16 (Ah: B x K; rsc: B norm scales), then the product with
 // both operands streamed straight into LDS (K a multiple of 64)

@@ -2598,7 +2598,8 @@ namespace ana {
 // the next stage's global loads in registers while the current one is
 // multiplied. ANA_BF16: v_mfma_f32_16x16x32_bf16 on the bf16 weights and
 // the activations rounded to bf16;
-// ANA_FAST_FP32: v_mfma_f32_16x16x4f32. Norm, residual and SiLU as in
+// ANA_FAST_FP32, for shapes the split tiles (gemm_split.hip) do not take:
+// v_mfma_f32_16x16x4f32. Norm, residual and SiLU as in
 // k_gemm_mfma (SiLU: tile rows 0..63 gate j, 64..127 up j).
 template <int WT>
 __global__ __launch_bounds__(256) void k_gemm_big(GemvArgs a) {

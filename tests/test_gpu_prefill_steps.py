@@ -45,3 +45,71 @@ def test_exact_ragged_steps(oracle, tmp_path, d, heads, arms):
             for l in range(c.layers):
                 assert np.array_equal(bits(dec.state(s, l)), bits(st.layer(l))), (i, l)
             assert np.array_equal(bits(lg[i]), bits(st.logits())), i
+
+
+def _rel(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+# (d, heads, MLP, sequences, tokens of the longest): the split tiles' remainders (rows
+# past a 16-, 64- and 128-row tile, 16-row weight tiles past the last full
+# one, 2 to 64 k steps, odd numbers among them) and, at the 115M's widths, each tile shape
+@pytest.mark.parametrize("d,heads,f,n,plen", [(64, 4, 192, 2, 70), (128, 4, 160, 3, 48), (256, 4, 1024, 5, 60),
+                                              (256, 4, 352, 8, 65), (768, 12, 2048, 17, 125), (768, 12, 2048, 64, 128)])
+def test_split_products(tmp_path, d, heads, f, n, plen):
+    """fast_fp32 prefill steps of 128 rows or more (k_split3, k_gemm_x3)
+    against the exact mode: every state and the logits. A product's parts
+    leave out less than one fp32 rounding, so what differs is the order of
+    fp32 sums: 1e-5 is about four times what k_gemm_big's fp32 products
+    show."""
+    c, path = _model(tmp_path, d, heads, True, ctx=256, layers=4 if d < 768 else 2, f=f, vocab=512)
+    lens = [max(1, plen - 3 * (i % 5)) for i in range(n)]
+    r = np.random.RandomState(d + f + n)
+    toks = [r.randint(0, c.vocab, k).astype(np.uint32) for k in lens]
+    seqs = list(range(n))
+    print(f"case split products d {d} f {f} rows {sum(lens)}", flush=True)
+    out = []
+    for mode in (ana_amd.FAST_FP32, ana_amd.EXACT_FP32):
+        with ana_amd.Decoder(path, max_seqs=n, prefill_chunk=128, numerics=mode) as dec:
+            dec.feeds_n(seqs, [0] * n, toks)
+            out.append((dec.logits(seqs), [dec.state(s, l) for s in (0, n - 1) for l in range(c.layers + 1)]))
+    assert _rel(out[0][0], out[1][0]) < 1e-5
+    for a, b in zip(out[0][1], out[1][1]):
+        assert _rel(a, b) < 1e-5
+    with ana_amd.Decoder(path, max_seqs=n, prefill_chunk=128, numerics=ana_amd.FAST_FP32) as dec:
+        ce = dec.score_n(seqs, [0] * n, toks)
+    with ana_amd.Decoder(path, max_seqs=n, prefill_chunk=128) as dec:
+        want = dec.score_n(seqs, [0] * n, toks)
+    assert _rel(np.concatenate(ce), np.concatenate(want)) < 1e-5
+
+
+def test_split_products_not_finite(tmp_path):
+    """A row that is not finite stays its own: its logits are NaN, as the
+    exact mode's, and the other sequences' what they are without it; a value
+    in the last binade (which rounds to infinity in bf16) counts as it does
+    in the exact mode."""
+    c = cf.Config(512, 256, 64, 192, 1, 4, True, True, True)
+    p = ckpt.init_params(c, "normal", 3, std=0.05, trained=True)
+    p[5 * c.d] = np.inf                    # token 5's embedding
+    p[6 * c.d] = np.float32(3.4e38)        # token 6's: its square overflows
+    path = str(tmp_path / "m.ftc2")
+    ckpt.write(path, c, p)
+    toks = [np.full(64, 9, np.uint32) for _ in range(3)]
+    with ana_amd.Decoder(path, max_seqs=3, prefill_chunk=64, numerics=ana_amd.FAST_FP32) as dec:
+        dec.feeds_n([0, 1, 2], [0] * 3, toks)
+        want = dec.logits([0, 1, 2])
+        for q in range(3):
+            dec.reset(q)
+        toks[1][-1] = 5
+        toks[2][-1] = 6
+        dec.feeds_n([0, 1, 2], [0] * 3, toks)
+        got = dec.logits([0, 1, 2])
+    with ana_amd.Decoder(path, max_seqs=3, prefill_chunk=64) as dec:
+        dec.feeds_n([0, 1, 2], [0] * 3, toks)
+        exact = dec.logits([0, 1, 2])
+    fin = np.delete(np.arange(c.vocab), [5, 6])   # (the tied head has those rows too)
+    got, want, exact = got[:, fin], want[:, fin], exact[:, fin]
+    assert np.isfinite(want).all() and np.array_equal(bits(got[0]), bits(want[0]))
+    assert np.isnan(got[1]).all() and np.isnan(exact[1]).all()
+    assert np.array_equal(np.isnan(got[2]), np.isnan(exact[2]))
