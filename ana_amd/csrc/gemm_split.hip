@@ -170,41 +170,39 @@ __global__ __launch_bounds__(WM * WN * 64) void k_gemm_x3(X3Args a) {
         __builtin_amdgcn_global_load_lds((const void*)(p + 512 * q), (lds_void*)(stage(B) + t * kBlk + 512 * q), 16, 0, 0);
     }
   };
-  f32x4_t acc[NI][MJ];
+  // the first parts' products in one sum, the five smaller ones (2^-8 of it
+  // and less) in another: the large sum is then rounded once a stage
+  f32x4_t acc[NI][MJ], low[NI][MJ];
 #pragma unroll
   for (int i = 0; i < NI; i++)
 #pragma unroll
-    for (int j = 0; j < MJ; j++) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-  // the fragments of the three parts, and the six products in two halves:
-  // `early` (1 1, 1 0, 0 1) as its reads land, `late` (2 0, 0 2, 0 0) held
-  // over the next stage's barrier, so that its matrix-core time covers that
-  // stage's first reads (all reads of a stage ahead of all its products left
-  // the matrix cores idle a fifth of the time: gate|up at 8192 rows 247 us)
-  bf16x8_t fw[3][NI], fa[3][MJ];
-  auto read = [&](auto B, int q) {
-    const __bf16* sa = stage(B) + wm * MJ * kBlk + 8 * lane + 512 * q;
-    const __bf16* sw = stage(B) + (AT + wn * NI) * kBlk + 8 * lane + 512 * q;
+    for (int j = 0; j < MJ; j++) acc[i][j] = low[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  // fragments of two parts at a time: the first parts' (fw0, fa0), and the
+  // second's, then the third's, in the same registers (fw, fa)
+  bf16x8_t fw0[NI], fa0[MJ], fw[NI], fa[MJ];
+  auto read_w = [&](auto B, int q, bf16x8_t (&f)[NI]) {
+    const __bf16* p = stage(B) + (AT + wn * NI) * kBlk + 8 * lane + 512 * q;
 #pragma unroll
-    for (int i = 0; i < NI; i++) fw[q][i] = *reinterpret_cast<const bf16x8_t*>(sw + i * kBlk);
-#pragma unroll
-    for (int j = 0; j < MJ; j++) fa[q][j] = *reinterpret_cast<const bf16x8_t*>(sa + j * kBlk);
+    for (int i = 0; i < NI; i++) f[i] = *reinterpret_cast<const bf16x8_t*>(p + i * kBlk);
   };
-  auto term = [&](int qw, int qa) {
+  auto read_a = [&](auto B, int q, bf16x8_t (&f)[MJ]) {
+    const __bf16* p = stage(B) + wm * MJ * kBlk + 8 * lane + 512 * q;
+#pragma unroll
+    for (int j = 0; j < MJ; j++) f[j] = *reinterpret_cast<const bf16x8_t*>(p + j * kBlk);
+  };
+  auto term = [&](f32x4_t (&c)[NI][MJ], const bf16x8_t (&w)[NI], const bf16x8_t (&x)[MJ]) {
 #pragma unroll
     for (int i = 0; i < NI; i++)
 #pragma unroll
-      for (int j = 0; j < MJ; j++)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[qw][i], fa[qa][j], acc[i][j], 0, 0, 0);
-  };
-  auto late = [&]() {
-    term(2, 0);
-    term(0, 2);
-    term(0, 0);
+      for (int j = 0; j < MJ; j++) c[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i], x[j], c[i][j], 0, 0, 0);
   };
   auto keep = [&]() { __builtin_amdgcn_sched_barrier(0); };   // (nothing moved across)
-  // this wave's loads of stage s are done and so are its reads of the other
-  // object; the barrier says so for every wave
+  // a stage: every read goes out a product or more before its use, the
+  // first ones before the last product of the stage before (held over the
+  // barrier), so the matrix cores work while the reads land
   auto step = [&](uint32_t s, auto B, auto Bn, auto first) {
+    // this wave's loads of stage s are done and so are its reads of the
+    // other object; the barrier says so for every wave
     keep();
     asm volatile("" ::: "memory");
     ANA_LGKMCNT0();
@@ -213,18 +211,27 @@ __global__ __launch_bounds__(WM * WN * 64) void k_gemm_x3(X3Args a) {
     asm volatile("" ::: "memory");
     keep();
     if (s + 1 < a.nk) issue(s + 1, Bn);
-    read(B, 1);
+    read_w(B, 1, fw);
+    read_a(B, 1, fa);
     keep();
-    if constexpr (!decltype(first)::value) late();
+    if constexpr (!decltype(first)::value) term(acc, fw0, fa0);
     keep();
-    read(B, 0);
+    read_a(B, 0, fa0);
+    read_w(B, 0, fw0);
     keep();
-    term(1, 1);
+    term(low, fw, fa);
     keep();
-    read(B, 2);
+    term(low, fw, fa0);
     keep();
-    term(1, 0);
-    term(0, 1);
+    read_w(B, 2, fw);
+    keep();
+    term(low, fw0, fa);
+    keep();
+    read_a(B, 2, fa);
+    keep();
+    term(low, fw, fa0);
+    keep();
+    term(low, fw0, fa);
     keep();
   };
   constexpr std::integral_constant<int, 0> S0{};
@@ -235,7 +242,11 @@ __global__ __launch_bounds__(WM * WN * 64) void k_gemm_x3(X3Args a) {
     step(s, S1, S0, std::false_type{});
     if (s + 1 < a.nk) step(s + 1, S0, S1, std::false_type{});
   }
-  late();
+  term(acc, fw0, fa0);
+#pragma unroll
+  for (int i = 0; i < NI; i++)
+#pragma unroll
+    for (int j = 0; j < MJ; j++) acc[i][j] += low[i][j];
   // this lane's results: row (mt0 + wm MJ + j) 16 + r16, columns
   // (nt0 + wn NI + i) 16 + 4 g4 .. + 3
   const uint32_t mt = mt0 + wm * MJ, nt = nt0 + wn * NI;
