@@ -157,6 +157,10 @@ static const uint32_t kGraphSteps = 8;
 // steps of every row d_out holds: ana_generate runs longer calls in pieces
 static const uint32_t kOutSteps = 1024;
 
+// rows a prefill step holds at most (more only by a larger prefill chunk or
+// more sequences than that)
+static const uint32_t kStepRows = 8192;
+
 static const size_t kProfMax = 16384;
 
 // bracket one launch with events on the context's stream
@@ -330,8 +334,13 @@ extern "C" int ana_open(const char* path, const ana_opts* opts, ana_ctx** out) {
   c->max_seqs = o.max_seqs;
   c->chunk = o.prefill_chunk;
   c->wb = std::max(c->max_seqs, c->chunk);
-  // a batched prefill's step holds every sequence's chunk, up to 8192 rows
-  c->rows = std::max<uint32_t>(c->wb, (uint32_t)std::min<uint64_t>((uint64_t)c->max_seqs * c->chunk, 8192));
+  // a prefill's step holds up to kStepRows rows: every sequence's chunk, or
+  // longer chunks of fewer sequences (step_chunk). Past the ring's wrap the
+  // steps keep to the context's chunk, and so do the fast attention's
+  // partials, which only those steps need for more than a few rows
+  const uint32_t wrap_rows =
+      std::max<uint32_t>(c->wb, (uint32_t)std::min<uint64_t>((uint64_t)c->max_seqs * c->chunk, kStepRows));
+  c->rows = std::max<uint32_t>(wrap_rows, (uint32_t)std::min<uint64_t>((uint64_t)c->max_seqs * ck.cfg.ctx, kStepRows));
   // a step holds at most kMaxSegs chunks (each at least one row), and so
   // at most rows / kGlaSub + seg_cap sub-chunks
   c->seg_cap = std::min({c->max_seqs, c->rows, kMaxSegs});
@@ -393,7 +402,7 @@ extern "C" int ana_open(const char* path, const ana_opts* opts, ana_ctx** out) {
   if (c->mode != ANA_EXACT_FP32) {
     // the fast kernels' scratch: attention partials for every row of a step,
     // the GLA scan's regions and tables
-    c->part_cap = attn_fast_part_floats(c->rows, cf.heads, cf.ctx, hd);
+    c->part_cap = attn_fast_part_floats(wrap_rows, cf.heads, cf.ctx, hd);
     if ((e = dalloc(&c->d_part, c->part_cap)) != hipSuccess ||
         (e = dalloc(&c->d_gla, gla_scan_floats(c->rows, c->gsub_cap, c->seg_cap, d, cf.heads))) != hipSuccess ||
         (e = dalloc(&c->d_gtab, c->gsub_cap)) != hipSuccess || (e = dalloc(&c->d_atab, c->atab_cap)) != hipSuccess)
@@ -1095,12 +1104,27 @@ extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint3
   return ANA_OK;
 }
 
-// dd.feeds (bend/Dense/Decode.bend:561-639) for n sequences at once. Step j
-// feeds tokens [jC, (j+1)C) of every sequence that has them (C the prefill
-// chunk): their rows go through each product together, the GLA and the
-// attention chunk by chunk, so each sequence ends as n separate dd.feeds
-// would leave it (bit for bit in ANA_EXACT_FP32: products are row-wise the
-// same for any number of rows).
+// dd.feeds (bend/Dense/Decode.bend:561-639) for n sequences at once. A step
+// feeds the next chunk of every sequence that has one: their rows go through
+// each product together, the GLA and the attention chunk by chunk, so each
+// sequence ends as n separate dd.feeds would leave it (bit for bit in
+// ANA_EXACT_FP32: products are row-wise the same for any number of rows).
+
+// A step's chunk, at least the context's prefill chunk: as many tokens of
+// each of the `live` sequences as fill the step's rows, since a step of few
+// rows leaves the chip idle (one 1919-token prompt at 115M, fast_fp32: 30
+// steps of 64 rows 25.1 ms, 3.9 ms in one). From kRunSeqs
+// sequences on the fast modes keep to kGlaRunMaxT tokens, where the GLA's
+// one workgroup a (head, chunk) fills the chip and moves a third of the
+// scan's bytes (64 us a layer at 8192 rows against 166 for the scan); fewer
+// sequences' longer chunks take the scan, whose sub-chunks run in parallel.
+constexpr uint32_t kRunSeqs = 16;
+static uint32_t step_chunk(const ana_ctx* c, uint32_t live) {
+  uint32_t C = c->rows / live;
+  if (fast_mode(c) && live >= kRunSeqs) C = std::min(C, kGlaRunMaxT);
+  return std::max(C & ~63u, c->chunk);
+}
+
 // the head over rows r0 .. r0 + g of X into SC, for scoring: in exact mode
 // the exact product (row-wise the bits of ana_logits' head), in the fast
 // modes the 128 x 128 matrix-core tiles
@@ -1136,7 +1160,6 @@ static int feeds_n(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, 
   std::vector<uint64_t> off(n), coff(n);
   std::vector<uint32_t> flen(n);
   uint64_t total = 0, ctot = 0;
-  uint32_t maxlen = 0;
   for (uint32_t i = 0; i < n; i++) {
     if (seq[i] >= c->max_seqs) return fail(c, ANA_EINVAL, "%s: sequence %u outside 0..%u", fn, seq[i], c->max_seqs - 1);
     if (seen[seq[i]]++) return fail(c, ANA_EINVAL, "%s: sequence %u listed twice", fn, seq[i]);
@@ -1145,7 +1168,6 @@ static int feeds_n(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, 
     flen[i] = ce ? (len[i] ? len[i] - 1 : 0) : len[i];
     coff[i] = ctot;
     ctot += ce ? flen[i] : 0;
-    maxlen = std::max(maxlen, flen[i]);
   }
   for (uint64_t i = 0; i < total; i++)
     if (toks[i] >= c->cfg.vocab) return fail(c, ANA_EINVAL, "%s: token %u outside the vocabulary", fn, toks[i]);
@@ -1192,10 +1214,24 @@ static int feeds_n(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, 
     cix.clear();
     return ANA_OK;
   };
-  for (uint32_t t0 = 0; t0 < maxlen; t0 += c->chunk) {
+  std::vector<uint32_t> at(n, 0);   // tokens fed
+  for (;;) {
+    uint32_t live = 0;
+    bool past = false;
     for (uint32_t i = 0; i < n; i++) {
+      if (at[i] >= flen[i]) continue;
+      live++;
+      past = past || (uint64_t)pos[i] + at[i] >= c->cfg.ctx;
+    }
+    if (!live) break;
+    const uint32_t C = past ? c->chunk : step_chunk(c, live);
+    for (uint32_t i = 0; i < n; i++) {
+      const uint32_t t0 = at[i];
       if (flen[i] <= t0) continue;
-      const uint32_t T = std::min(c->chunk, flen[i] - t0);
+      uint32_t T = std::min(C, flen[i] - t0);
+      // up to the ring's wrap in one chunk, the rest past it
+      const uint64_t p0 = (uint64_t)pos[i] + t0;
+      if (p0 < c->cfg.ctx) T = (uint32_t)std::min<uint64_t>(T, c->cfg.ctx - p0);
       if (rows.size() + T > c->rows || segs.size() == c->seg_cap)
         if (int r = flush()) return r;
       segs.push_back(Seg{seq[i], pos[i] + t0, (uint32_t)rows.size(), T});
@@ -1205,6 +1241,7 @@ static int feeds_n(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, 
           tg.push_back(toks[off[i] + t + 1]);
           cix.push_back(coff[i] + t);
         }
+      at[i] = t0 + T;
     }
     // the next step's chunks start from the states this step leaves
     if (int r = flush()) return r;

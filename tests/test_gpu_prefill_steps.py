@@ -113,3 +113,47 @@ def test_split_products_not_finite(tmp_path):
     assert np.isfinite(want).all() and np.array_equal(bits(got[0]), bits(want[0]))
     assert np.isnan(got[1]).all() and np.isnan(exact[1]).all()
     assert np.array_equal(np.isnan(got[2]), np.isnan(exact[2]))
+
+
+@pytest.mark.parametrize("chunk", [1, 16, 64])
+def test_exact_steps_over_the_wrap(oracle, tmp_path, chunk):
+    """step_chunk's steps: a step's chunk runs up to the ring's wrap (64
+    slots) whatever the context's chunk, and keeps to it past the wrap; one
+    sequence, then three at once from different positions; bit for bit."""
+    c, path = _model(tmp_path, 64, 4, True)
+    m = oracle.Model(path)
+    r = np.random.RandomState(chunk)
+    toks = [r.randint(0, c.vocab, k).astype(np.uint32) for k in (150, 40, 23)]
+    more = [r.randint(0, c.vocab, k).astype(np.uint32) for k in (9, 31, 41)]
+    print(f"case exact steps over the wrap, chunk {chunk}", flush=True)
+    with ana_amd.Decoder(path, max_seqs=3, prefill_chunk=chunk) as dec:
+        for i in range(3):
+            dec.feeds(i, 0, toks[i])
+        dec.feeds_n([2, 0, 1], [23, 150, 40], [more[2], more[0], more[1]])
+        for i in range(3):
+            st = oracle.State(m)
+            st.feeds(0, np.concatenate([toks[i], more[i]]))
+            for l in range(c.layers):
+                assert np.array_equal(bits(dec.state(i, l)), bits(st.layer(l))), (i, l)
+            assert np.array_equal(bits(dec.logits([i])[0]), bits(st.logits())), i
+
+
+@pytest.mark.parametrize("n,plen", [(1, 300), (3, 300), (15, 280), (16, 300), (40, 260)])
+def test_fast_steps(tmp_path, n, plen):
+    """step_chunk's longer chunks in fast_fp32, on both sides of its rules
+    (the GLA scan for fewer than 16 sequences, chunks of at most 256 tokens
+    from there, more rows than a step holds) against the exact mode, as
+    test_split_products holds them."""
+    c, path = _model(tmp_path, 64, 4, True, ctx=512, f=192)
+    r = np.random.RandomState(n)
+    toks = [r.randint(0, c.vocab, plen - i % 7).astype(np.uint32) for i in range(n)]
+    seqs = list(range(n))
+    print(f"case fast steps n {n}", flush=True)
+    out = []
+    for mode in (ana_amd.FAST_FP32, ana_amd.EXACT_FP32):
+        with ana_amd.Decoder(path, max_seqs=n, numerics=mode) as dec:
+            dec.feeds_n(seqs, [0] * n, toks)
+            out.append((dec.logits(seqs), [dec.state(s, l) for s in (0, n - 1) for l in range(c.layers + 1)]))
+    assert _rel(out[0][0], out[1][0]) < 1e-5
+    for a, b in zip(out[0][1], out[1][1]):
+        assert _rel(a, b) < 1e-5
