@@ -976,7 +976,7 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
           HIPCHK(c, launch_attn_fast(a, c->st));
         } else if (fast_mode(c)) {
           a.part = c->d_part;
-          HIPCHK(c, launch_attn_rows(a, c->attn_split || cf.ctx > kAttnRowsMaxCtx, c->st));
+          HIPCHK(c, launch_attn_rows(a, c->attn_split, c->st));
         } else {
           HIPCHK(c, launch_attn(a, c->st));
         }

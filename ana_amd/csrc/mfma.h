@@ -1,12 +1,24 @@
-// Matrix-core helpers shared by the fast product kernels (gfx950): operand
+// Helpers shared by the fast kernels (gfx950): compile-time loops, operand
 // vectors, the LDS address type of global_load_lds, explicit wait counts,
 // the SiLU of the gate|up epilogues and the XCD-grouped tile order.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
+#include <utility>
 
 namespace ana {
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>), in order
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_(f, std::make_integer_sequence<int, N>{});
+}
 
 // MFMA operand and accumulator vectors
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
