@@ -536,6 +536,17 @@ static bool reads_bf16(const ana_ctx* c, const GemvArgs& g) {
 static const uint32_t kBigB = 128;   // prefill steps of this many rows or more take the big tiles
 static hipError_t launch_x3(ana_ctx* c, const GemvArgs& g, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 
+// an exact product of more than kSmallB rows reads its input normed: the
+// norm's rows into XN
+static hipError_t norm_first(ana_ctx* c, GemvArgs& g) {
+  if (!g.ng || g.B <= kSmallB) return hipSuccess;
+  if (g.ldx != g.K || g.K != c->cfg.d || g.B > c->rows) return hipErrorInvalidValue;
+  const hipError_t e = launch_rmsnorm(g.X, g.ng, g.K, g.B, c->XN, c->st);
+  g.X = c->XN;
+  g.ng = nullptr;
+  return e;
+}
+
 // next_gain: the norm gain of the product that reads this one's outputs
 // next (a prefill step's residual products), for a producer-side bf16 copy
 static hipError_t gemv_timed(ana_ctx* c, const GemvArgs& g0, uint32_t kind, bool chunk = false,
@@ -617,8 +628,10 @@ static hipError_t gemv_timed(ana_ctx* c, const GemvArgs& g0, uint32_t kind, bool
     return launch_gemm_mfma(g, c->st, ps.start(), ps.stop());
   }
   if (hh_only) return hipErrorInvalidValue;
+  GemvArgs g = g0;
+  if (const hipError_t e = norm_first(c, g)) return e;
   ProfScope ps(c, kind, gemv_bytes(g0), true);
-  return launch_gemv(g0, c->st, ps.start(), ps.stop());
+  return launch_gemv(g, c->st, ps.start(), ps.stop());
 }
 
 static GemvArgs gemv1(const float* X, uint32_t ldx, uint32_t K, const float* W, uint32_t rows,
@@ -1144,6 +1157,7 @@ static int score_head(ana_ctx* c, uint32_t r0, uint32_t g) {
     else
       HIPCHK(c, launch_gemm_big(h, c->st));
   } else {
+    HIPCHK(c, norm_first(c, h));
     HIPCHK(c, launch_gemv(h, c->st));
   }
   return ANA_OK;

@@ -14,6 +14,7 @@
 #include <stdlib.h>
 
 #include "ana_internal.h"
+#include "mfma.h"
 #include "numerics.h"
 
 #pragma clang fp contract(off)
@@ -196,141 +197,81 @@ __global__ __launch_bounds__(256) void k_gemv_small(GemvArgs a, uint32_t R, uint
 }
 
 // Larger batches (prefill chunks, batched decode): a tile of TR weight rows
-// x TB batch rows per workgroup; thread (ti, tj) owns RI x BJ chains (rows
-// ti*RI.., batch rows tj*BJ..). The K axis goes in chunks of KC. Every
-// thread moves NL float4 of each chunk (weights and activations, coalesced
-// along k) through a ring of D register sets, so D-1 chunks are in flight
-// from HBM while one is added; a chunk is stored k-major into one of two
-// LDS buffers, and each chain multiplies and adds in q order out of LDS:
-// bulk.c's ft_gemm_loop, one lane per output. With `ng` the workgroup first
-// runs M.norm's sum of squares for its TB rows (one in-order chain per row,
-// while the first chunks are in flight) and stages (x * rs) * g.
+// x TB batch rows per workgroup; thread (ti, tj) owns RI x BJ chains (weight
+// rows ti, ti + NI, .., batch rows tj, tj + NJ, ..: a wave's reads of one
+// k4 are then consecutive float4s, without bank conflicts). The K axis goes
+// in chunks of KC. Every thread moves NL float4 of each chunk (weights and
+// activations, coalesced along k) through a ring of D register sets, so D-1
+// chunks are in flight from HBM while one is added; a chunk is stored
+// k-major into one of two LDS buffers, and each chain multiplies and adds in
+// q order out of LDS: bulk.c's ft_gemm_loop, one lane per output. The input
+// comes normed (k_rmsnorm): with the norm inside, every column tile formed
+// its rows' sums of squares again, a chain of K adds before its first
+// product, and staged three more operations a value (q|k|v|z at 64 rows
+// 33.2 us against 18.3 and 5.4 for the norm, at 2048 rows 351 against 214 and
+// 10). Bound by its two operations a term, a multiply and an add: 246 us for
+// the 2048-row product at one wave operation in four cycles of 2.4 GHz.
 template <int TR, int TB, int RI, int BJ, int KC, int D, int G>
 __global__ __launch_bounds__(256) void k_gemm_exact(GemvArgs a) {
   constexpr int NJ = TB / BJ, NI = TR / RI;
   static_assert(NI * NJ == 256, "one chain block per thread");
   constexpr int K4 = KC / 4;
-  constexpr int LW = TR * K4, LX = TB * K4, NL = (LW + LX + 255) / 256;
+  constexpr int LW = TR * K4, LX = TB * K4, NL = (LW + LX) / 256;
+  static_assert((LW + LX) % 256 == 0, "whole float4s a thread");
   static_assert(K4 % (2 * G) == 0, "whole read groups per chunk");
-  __shared__ float4 Ws[2][K4][TR + 1];
-  __shared__ float4 Xs[2][K4][TB + 1];
-  __shared__ float rs[TB];
+  // a chunk k-major: the weight rows' columns, then (from XC) the batch rows'
+  constexpr int XC = TR + 1;
+  __shared__ f32x4_t Cs[2][K4][XC + TB + 1];
   __shared__ float outs[TB][TR + 1];
   const uint32_t tid = threadIdx.x;
   const uint32_t tj = tid % NJ, ti = tid / NJ;
   const uint32_t b0 = blockIdx.y * TB;
   const uint32_t nb = min((uint32_t)TB, a.B - b0);
   const Segs sgs(a);
-  const bool norm = a.ng != nullptr;
   const uint32_t nch = (a.K + KC - 1) / KC;
 
   // the NL float4 this thread moves per chunk: item i = tid + 256 j;
   // i < LW: weight row i / K4, k4 = i % K4; else batch row (i-LW) / K4
+  // (native vectors: as HIP's float4, a struct copied whole between global
+  // memory and LDS, the ring was kept in scratch memory)
   const float* src[NL];
-  uint32_t dk4[NL], drow[NL];
-  bool ok[NL];
-#pragma unroll
-  for (int j = 0; j < NL; j++) {
+  uint32_t dk4[NL], dcol[NL];
+  static_for<NL>([&](auto J) {
+    constexpr int j = decltype(J)::value;
     const uint32_t i = tid + 256 * j;
+    dk4[j] = i % K4;
     if (i < (uint32_t)LW) {
-      const uint32_t r = i / K4;
       const float* w;
       uint32_t sg, lr;
-      ok[j] = sgs.row(TR, blockIdx.x, r, &w, &sg, &lr);
-      src[j] = ok[j] ? w : sgs.W0;
-      dk4[j] = i % K4;
-      drow[j] = r;
+      const bool ok = sgs.row(TR, blockIdx.x, i / K4, &w, &sg, &lr);
+      src[j] = ok ? w : sgs.W0;
+      dcol[j] = i / K4;
     } else {
       const uint32_t b = (i - LW) / K4;
-      ok[j] = b < nb && i < (uint32_t)(LW + LX);
-      src[j] = a.X + (size_t)(b0 + (ok[j] ? b : 0)) * a.ldx;
-      dk4[j] = (i - LW) % K4;
-      drow[j] = b;
+      src[j] = a.X + (size_t)(b0 + (b < nb ? b : 0)) * a.ldx;
+      dcol[j] = XC + b;
     }
-  }
-  float4 v[D][NL];
-  auto load = [&](float4 (&r)[NL], uint32_t c) {
-#pragma unroll
-    for (int j = 0; j < NL; j++) {
+  });
+  f32x4_t v[D][NL];
+  auto load = [&](auto U, uint32_t c) {
+    static_for<NL>([&](auto J) {
+      constexpr int u = decltype(U)::value, j = decltype(J)::value;
       const uint32_t q = c * KC + 4 * dk4[j];
-      const bool in = ok[j] && q < a.K;
       // an unconditional load from a clamped address, so that it stays in
-      // flight; items out of range are never added or stored, so they are
-      // not zeroed (writing the destination would wait for the load)
-      r[j] = *reinterpret_cast<const float4*>(src[j] + (in ? q : 0));
-    }
+      // flight; values past K or the rows are never added or stored
+      v[u][j] = *reinterpret_cast<const f32x4_t*>(src[j] + (q < a.K ? q : 0));
+    });
   };
-  auto store = [&](const float4 (&r)[NL], int buf, uint32_t c) {
-#pragma unroll
-    for (int j = 0; j < NL; j++) {
-      const uint32_t i = tid + 256 * j;
-      if (i < (uint32_t)LW) {
-        Ws[buf][dk4[j]][drow[j]] = r[j];
-      } else if (i < (uint32_t)(LW + LX)) {
-        float4 x = r[j];
-        if (norm) {
-          const uint32_t q = c * KC + 4 * dk4[j];
-          const float sc = rs[drow[j]];
-          const float4 g = *reinterpret_cast<const float4*>(a.ng + (q < a.K ? q : 0));
-          x.x = (x.x * sc) * g.x;
-          x.y = (x.y * sc) * g.y;
-          x.z = (x.z * sc) * g.z;
-          x.w = (x.w * sc) * g.w;
-        }
-        Xs[buf][dk4[j]][drow[j]] = x;
-      }
-    }
+  auto store = [&](auto U, int buf) {
+    static_for<NL>([&](auto J) {
+      constexpr int u = decltype(U)::value, j = decltype(J)::value;
+      Cs[buf][dk4[j]][dcol[j]] = v[u][j];
+    });
   };
-
-#pragma unroll
-  for (int u = 0; u < D; u++)
-    if ((uint32_t)u < nch) load(v[u], u);
-  if (norm) {
-    // M.norm (bend/Dense/Model.bend:27-30): ss = sum_q x_q * x_q in order,
-    // one chain per batch row over the activations staged chunk by chunk
-    // through the X buffers (the weights of the first chunks keep arriving)
-    constexpr int PX = (LX + 255) / 256;
-    float4 xr[2][PX];
-    auto xload = [&](float4 (&r)[PX], uint32_t c) {
-#pragma unroll
-      for (int j = 0; j < PX; j++) {
-        const uint32_t i = tid + 256 * j, b = i / K4, q = c * KC + 4 * (i % K4);
-        const bool in = i < (uint32_t)LX && b < nb && q < a.K;
-        r[j] = *reinterpret_cast<const float4*>(a.X + (size_t)(b0 + (in ? b : 0)) * a.ldx + (in ? q : 0));
-      }
-    };
-    auto xstore = [&](const float4 (&r)[PX], int buf) {
-#pragma unroll
-      for (int j = 0; j < PX; j++) {
-        const uint32_t i = tid + 256 * j;
-        if (i < (uint32_t)LX) Xs[buf][i % K4][i / K4] = r[j];
-      }
-    };
-    float ss = 0.0f;
-    xload(xr[0], 0);
-    xstore(xr[0], 0);
-    __syncthreads();
-    for (uint32_t c = 0; c < nch; c++) {
-      const int bf = c & 1;
-      if (c + 1 < nch) xload(xr[1], c + 1);
-      if (tid < (uint32_t)TB) {
-        const uint32_t n4 = min((uint32_t)K4, (a.K - c * KC) >> 2);
-#pragma unroll 8
-        for (uint32_t k4 = 0; k4 < n4; k4++) {
-          const float4 x = Xs[bf][k4][tid];
-          ss = ss + x.x * x.x;
-          ss = ss + x.y * x.y;
-          ss = ss + x.z * x.z;
-          ss = ss + x.w * x.w;
-        }
-      }
-      if (c + 1 < nch) xstore(xr[1], bf ^ 1);
-      __syncthreads();
-    }
-    if (tid < (uint32_t)TB) rs[tid] = ex_rms_scale(ss, (float)a.K);
-    __syncthreads();
-  }
-  store(v[0], 0, 0);
+  static_for<D>([&](auto U) {
+    if ((uint32_t)decltype(U)::value < nch) load(U, decltype(U)::value);
+  });
+  store(std::integral_constant<int, 0>{}, 0);
   __syncthreads();
 
   float s[RI][BJ];
@@ -339,7 +280,7 @@ __global__ __launch_bounds__(256) void k_gemm_exact(GemvArgs a) {
 #pragma unroll
     for (int j = 0; j < BJ; j++) s[i][j] = 0.0f;
 
-  auto step = [&](const float4 (&w)[RI], const float4 (&x)[BJ]) {
+  auto step = [&](const f32x4_t (&w)[RI], const f32x4_t (&x)[BJ]) {
 #pragma unroll
     for (int i = 0; i < RI; i++)
 #pragma unroll
@@ -360,14 +301,14 @@ __global__ __launch_bounds__(256) void k_gemm_exact(GemvArgs a) {
   // one chunk out of LDS buffer buf: groups of G k4 steps in two register
   // sets, the next group's reads issued before the current group adds
   auto chunk = [&](int buf, uint32_t n4) {
-    float4 wa[G][RI], xa[G][BJ], wb[G][RI], xb[G][BJ];
-    auto rd = [&](float4 (&w)[G][RI], float4 (&x)[G][BJ], uint32_t kb) {
+    f32x4_t wa[G][RI], xa[G][BJ], wb[G][RI], xb[G][BJ];
+    auto rd = [&](f32x4_t (&w)[G][RI], f32x4_t (&x)[G][BJ], uint32_t kb) {
 #pragma unroll
       for (int u = 0; u < G; u++) {
 #pragma unroll
-        for (int i = 0; i < RI; i++) w[u][i] = Ws[buf][kb + u][ti * RI + i];
+        for (int i = 0; i < RI; i++) w[u][i] = Cs[buf][kb + u][ti + NI * i];
 #pragma unroll
-        for (int j = 0; j < BJ; j++) x[u][j] = Xs[buf][kb + u][tj * BJ + j];
+        for (int j = 0; j < BJ; j++) x[u][j] = Cs[buf][kb + u][XC + tj + NJ * j];
       }
     };
     uint32_t k4 = 0;
@@ -384,45 +325,44 @@ __global__ __launch_bounds__(256) void k_gemm_exact(GemvArgs a) {
       }
     }
     for (; k4 < n4; k4++) {
-      float4 w[RI], x[BJ];
+      f32x4_t w[RI], x[BJ];
 #pragma unroll
-      for (int i = 0; i < RI; i++) w[i] = Ws[buf][k4][ti * RI + i];
+      for (int i = 0; i < RI; i++) w[i] = Cs[buf][k4][ti + NI * i];
 #pragma unroll
-      for (int j = 0; j < BJ; j++) x[j] = Xs[buf][k4][tj * BJ + j];
+      for (int j = 0; j < BJ; j++) x[j] = Cs[buf][k4][XC + tj + NJ * j];
       step(w, x);
     }
   };
 
   // chunk c sits in LDS buffer c & 1 and (before that) in register set c % D
-  for (uint32_t c0 = 0; c0 < nch; c0 += D) {
-#pragma unroll
-    for (int u = 0; u < D; u++) {
+  for (uint32_t c0 = 0; c0 < nch; c0 += D)
+    static_for<D>([&](auto U) {
+      constexpr int u = decltype(U)::value;
       const uint32_t c = c0 + u;
       if (c < nch) {
         chunk(c & 1, min((uint32_t)K4, (a.K - c * KC) >> 2));
-        if (c + 1 < nch) store(v[(u + 1) % D], (c + 1) & 1, c + 1);
-        if (c + D < nch) load(v[u], c + D);
+        if (c + 1 < nch) store(std::integral_constant<int, (u + 1) % D>{}, (c + 1) & 1);
+        if (c + D < nch) load(U, c + D);
         __syncthreads();
       }
-    }
-  }
+    });
 
   if (a.mode == GM_SILU) {
     // gate rows are tile rows [0, TR/2), their up rows TR/2 further
 #pragma unroll
     for (int i = 0; i < RI; i++)
 #pragma unroll
-      for (int j = 0; j < BJ; j++) outs[tj * BJ + j][ti * RI + i] = s[i][j];
+      for (int j = 0; j < BJ; j++) outs[tj + NJ * j][ti + NI * i] = s[i][j];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < RI; i++) {
-      const uint32_t r = ti * RI + i;
+      const uint32_t r = ti + NI * i;
       const float* w;
       uint32_t sg, lr;
       if (r < (uint32_t)TR / 2 && sgs.row(TR, blockIdx.x, r, &w, &sg, &lr)) {
 #pragma unroll
         for (int j = 0; j < BJ; j++) {
-          const uint32_t b = tj * BJ + j;
+          const uint32_t b = tj + NJ * j;
           if (b < nb)
             a.seg[0].Y[(size_t)(b0 + b) * a.seg[0].ldy + lr] = ex_silu(s[i][j]) * outs[b][r + TR / 2];
         }
@@ -434,10 +374,10 @@ __global__ __launch_bounds__(256) void k_gemm_exact(GemvArgs a) {
   for (int i = 0; i < RI; i++) {
     const float* w;
     uint32_t sg, lr;
-    if (sgs.row(TR, blockIdx.x, ti * RI + i, &w, &sg, &lr)) {
+    if (sgs.row(TR, blockIdx.x, ti + NI * i, &w, &sg, &lr)) {
 #pragma unroll
       for (int j = 0; j < BJ; j++) {
-        const uint32_t b = tj * BJ + j;
+        const uint32_t b = tj + NJ * j;
         if (b < nb) gemv_store(a, sg, lr, b0 + b, s[i][j]);
       }
     }
@@ -467,6 +407,14 @@ static const uint32_t kRmax = env_u32("ANA_GEMV_RMAX", 64);
     if (E0) hipExtLaunchKernelGGL(K, GRID, BLOCK, LDS, ST, E0, E1, 0, __VA_ARGS__);      \
     else hipLaunchKernelGGL(K, GRID, BLOCK, LDS, ST, __VA_ARGS__);                      \
   } while (0)
+
+static uint32_t device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+    return 256;
+  return (uint32_t)n;
+}
 
 hipError_t launch_gemv(const GemvArgs& a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   const uint32_t rows = a.mode == GM_SILU ? 2 * a.seg[0].rows
@@ -504,15 +452,25 @@ hipError_t launch_gemv(const GemvArgs& a, hipStream_t st, hipEvent_t e0, hipEven
     return hipGetLastError();
   }
   if (a.amax) return hipErrorInvalidValue;  // batched products store logits instead
-  if (a.ng && (a.K & 3)) return hipErrorInvalidValue;
-  // one chain per thread over 16 x 16 tiles while that still leaves a few
-  // workgroups per CU; 2 x 2 chains per thread over 32 x 32 tiles beyond
-  const bool big = (uint64_t)rows * a.B >= 256ull * 1024;
-  const uint32_t TR = big ? 32 : 16, TB = TR;
+  if (a.ng) return hipErrorInvalidValue;    // (their inputs come normed: launch_rmsnorm)
+  // the tile that finishes first by what the shapes measured at K = 768 (us,
+  // w workgroups a CU): 16 x 16, one chain a thread, for the fewest rows (Wo
+  // at 64 rows 12.1, 32 x 32 25.1); 32 x 32, 2 x 2 chains, from about two
+  // workgroups a CU (q|k|v|z at 128 rows 33.5 and 28.9); 64 x 64, 4 x 4
+  // chains, half the LDS reads a chain, where they too fill the CUs
+  // (gate|up at 2048 rows 299 and 264)
+  static const uint32_t cus = device_cus();
+  auto per_cu = [&](uint32_t t) { return (float)((((uint64_t)(rows + t - 1) / t) * ((a.B + t - 1) / t) + cus - 1) / cus); };
+  const float w16 = per_cu(16), w32 = per_cu(32), w64 = per_cu(64);
+  const float c16 = fmaxf(12.0f, 5.3f * w16);
+  const float c32 = w32 <= 1.0f ? 25.0f : fmaxf(28.5f, 9.6f * w32 + 8.0f);
+  const float c64 = w64 <= 1.0f ? 73.0f : fmaxf(79.0f, 33.0f * w64);
+  const uint32_t TR = c64 < c32 && c64 < c16 ? 64 : c32 < c16 ? 32 : 16;
   const uint32_t per = a.mode == GM_SILU ? TR / 2 : TR;
   const uint32_t tiles = a.mode == GM_SILU ? (a.seg[0].rows + per - 1) / per : (rows + per - 1) / per;
-  dim3 grid(tiles, (a.B + TB - 1) / TB);
-  if (big) ANA_LAUNCH((k_gemm_exact<32, 32, 2, 2, 64, 3, 1>), grid, dim3(256), 0, st, e0, e1, a);
+  dim3 grid(tiles, (a.B + TR - 1) / TR);
+  if (TR == 64) ANA_LAUNCH((k_gemm_exact<64, 64, 4, 4, 16, 3, 1>), grid, dim3(256), 0, st, e0, e1, a);
+  else if (TR == 32) ANA_LAUNCH((k_gemm_exact<32, 32, 2, 2, 64, 3, 1>), grid, dim3(256), 0, st, e0, e1, a);
   else ANA_LAUNCH((k_gemm_exact<16, 16, 1, 1, 128, 4, 4>), grid, dim3(256), 0, st, e0, e1, a);
   return hipGetLastError();
 }
@@ -528,7 +486,12 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float* __restrict__ X,
   const float4* x = reinterpret_cast<const float4*>(X + (size_t)blockIdx.x * d);
   for (uint32_t i = tid; i < d4; i += 256) xs4[i] = x[i];
   __syncthreads();
-  if (tid == 0) scale = ex_rms_scale(chain_sumsq_lds(0.0f, reinterpret_cast<const float*>(xs4), d), (float)d);
+  // (every lane of a wave runs the chain: a wave with its other lanes off
+  // takes twice the time an add)
+  if (tid < 64) {
+    const float t = ex_rms_scale(chain_sumsq_lds(0.0f, reinterpret_cast<const float*>(xs4), d), (float)d);
+    if (tid == 0) scale = t;
+  }
   __syncthreads();
   const float sc = scale;
   const float4* g4 = reinterpret_cast<const float4*>(g);
