@@ -306,13 +306,17 @@ uint32_t w_rows(const GemvArgs& a) {
   return a.mode == GM_SILU ? 2 * a.seg[0].rows : a.seg[0].rows + (a.nseg > 1 ? a.seg[1].rows : 0);
 }
 
-// 96 columns a tile where 128 leave a round part empty: Wo and down at 8192
-// rows are 192 workgroups of 128 columns on 256 CUs, 256 of 96.
-// The tile for a product: the one whose rounds of workgroups cost least (a
-// tile's area, times what that shape costs an area unit against the largest
-// tile, times the rounds the CUs take; `per` workgroups share a CU).
-struct Tile { uint32_t bm, bn, per; float unit; };
-constexpr Tile kTiles[] = {{256, 128, 1, 1.0f}, {256, 96, 1, 1.0f}, {128, 128, 1, 1.2f}, {64, 64, 3, 1.6f}};
+// The tile for a product: the one whose workgroups finish first by what the
+// shapes measured at K = 768 (us; every one grows with K alike). `per`
+// workgroups share a CU: a full round of them takes `round`, a last round
+// of one or two a CU part[1] or part[2]. So 96 columns where 128 leave a
+// round part empty (Wo at 8192 rows: 192 workgroups of 256 x 128 on 256 CUs
+// 62 us, 256 of 256 x 96 54 us), and 64 x 64 where the larger ones leave CUs
+// idle (Wo at 1919 rows 43 us with 256 x 96, 31 with 128 x 128, 20 with
+// 64 x 64; gate|up at 256 rows 48, 28 and 17).
+struct Tile { uint32_t bm, bn, per; float round, part[3]; };
+constexpr Tile kTiles[] = {{256, 128, 1, 57.0f, {}}, {256, 96, 1, 47.0f, {}}, {128, 128, 1, 33.0f, {}},
+                           {64, 64, 3, 29.0f, {0.0f, 15.0f, 20.0f}}};
 
 int pick_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus) {
   int best = 0;
@@ -320,8 +324,8 @@ int pick_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus) {
   for (int t = 0; t < 4; t++) {
     const Tile& k = kTiles[t];
     if (silu && k.bn == 96) continue;
-    const uint32_t wgs = (B + k.bm - 1) / k.bm * ((rows + k.bn - 1) / k.bn), slots = cus * k.per;
-    const float cost = (float)((wgs + slots - 1) / slots) * (float)(k.bm * k.bn * k.per) * k.unit;
+    const uint32_t wgs = (B + k.bm - 1) / k.bm * ((rows + k.bn - 1) / k.bn), w = (wgs + cus - 1) / cus;
+    const float cost = (float)(w / k.per) * k.round + k.part[w % k.per];
     if (t == 0 || cost < least) {
       best = t;
       least = cost;
