@@ -989,7 +989,7 @@ static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_
           HIPCHK(c, launch_attn_fast(a, c->st));
         } else if (fast_mode(c)) {
           a.part = c->d_part;
-          HIPCHK(c, launch_attn_rows(a, c->attn_split, c->st));
+          HIPCHK(c, launch_attn_rows(a, c->attn_split || cf.ctx > kAttnRowsMaxCtx, c->st));
         } else {
           HIPCHK(c, launch_attn(a, c->st));
         }
@@ -1132,7 +1132,12 @@ extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint3
 // scan's bytes (64 us a layer at 8192 rows against 166 for the scan); fewer
 // sequences' longer chunks take the scan, whose sub-chunks run in parallel.
 constexpr uint32_t kRunSeqs = 16;
-static uint32_t step_chunk(const ana_ctx* c, uint32_t live) {
+// ANA_BF16 calls of kRunSeqs sequences or more keep the context's chunk: a
+// chunk's length moves where activations round to bf16, and picks near a tie
+// follow (such callers set the chunk for speed themselves: 64 prompts of 512
+// tokens run 1.97M tok/s at 64, 2.64M at 128).
+static uint32_t step_chunk(const ana_ctx* c, uint32_t n, uint32_t live) {
+  if (c->mode == ANA_BF16 && n >= kRunSeqs) return c->chunk;
   uint32_t C = c->rows / live;
   if (fast_mode(c) && live >= kRunSeqs) C = std::min(C, kGlaRunMaxT);
   return std::max(C & ~63u, c->chunk);
@@ -1238,7 +1243,7 @@ static int feeds_n(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, 
       past = past || (uint64_t)pos[i] + at[i] >= c->cfg.ctx;
     }
     if (!live) break;
-    const uint32_t C = past ? c->chunk : step_chunk(c, live);
+    const uint32_t C = past ? c->chunk : step_chunk(c, n, live);
     for (uint32_t i = 0; i < n; i++) {
       const uint32_t t0 = at[i];
       if (flen[i] <= t0) continue;

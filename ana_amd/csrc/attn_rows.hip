@@ -7,44 +7,27 @@
 
 namespace ana {
 
-// the sum over each group of L consecutive lanes (L = 4, 8 or 16), in every
-// lane of the group, by DPP
-template <int L>
-__device__ __forceinline__ float lanes_sum(float v) {
-  static_assert(L == 4 || L == 8 || L == 16, "a quad, a half row or a row");
-  v += dpp<0xB1>(v);
-  v += dpp<0x4E>(v);
-  if constexpr (L >= 8) v += dpp<0x141>(v);
-  if constexpr (L >= 16) v += dpp<0x140>(v);
-  return v;
-}
-
 // Decode attention of more than kSmallB rows in the fast modes: one
 // workgroup per (head, row) over the row's live slots 0 .. npos. The row's
 // k (qk-normed when on) and v go to its slot first; its own slot's score
-// and product come from registers. A slot is L = HD / 4 lanes (a float4 of
-// its K and V row each, so a slot's row is one 16 L-byte piece), the
-// workgroup G = 256 / L slot groups, a stage U slots a group. A stage's K
-// and V come in together, D stages in flight in registers from before the
-// row's q is known, and each group keeps a running max m, sum l and sum
-// e V of its own (scaled once a stage), so no barrier and no wait but the
-// loads' stand between the stages; the groups meet in LDS at the end. Bound
-// by the K and V rows' bytes: 59 MB a layer at B = 64 and ~150 slots 18.5 us,
-// 379 MB at B = 32 and ~1900 in 256-slot pieces 77.2 us with the combine's
-// 4.8 (two passes over the window, the scores in LDS between them: 19.4,
-// 78.0 and 6.5; a kernel that only reads those rows, in pieces of 256 bytes
-// or of 1 KB: 14.7 and 67). U = 2 and D = 3 against 4 and 3: fewer
-// registers, 18.5 against 20.2 us. With
-// a split grid (gridDim.z > 1) workgroup z takes slots z SL .. z SL + SL - 1
-// of the live ones (SL = kRowsSplit), and leaves its max m, its sum l = sum e
-// and its o = sum e V (e = exp(sc s - m), no sink) in part for
-// k_attn_rows_comb.
+// and product take them from LDS. A slot is L = HD / 4 lanes (a float4 of
+// its K or V row each, so a slot's row is one 16 L-byte piece), the
+// workgroup G = 256 / L slot groups, and a trip U slots a group, the next
+// trip's loads in flight while one computes. Pass 1 keeps sc*s in LDS
+// (ctx floats, dynamic); the max (with the sink) and the denominator come
+// from wave and block reductions; pass 2 sums e*V per lane over its slots
+// for its four columns, and the G slot groups meet in LDS. With a split
+// grid (gridDim.z > 1) workgroup z takes slots z SL .. z SL + SL - 1 of the
+// live ones (SL = kRowsSplit), and leaves its max m, its sum l = sum e and
+// its o = sum e V (e = exp(sc s - m), no sink) in part for k_attn_rows_comb.
 template <int HD>
 __global__ __launch_bounds__(256) void k_attn_rows(AttnArgs a) {
-  constexpr int L = HD / 4, G = 256 / L, U = 2, D = 3, ST = U * G;
-  constexpr float kLow = -3.0e38f;   // below every score, and finite (exp(-inf - kLow) is 0)
-  __shared__ float nrm[2], ms[G], ls[G], ws[G];
-  __shared__ __align__(16) float kv[2][HD];
+  constexpr int L = HD / 4, G = 256 / L, U = 4;
+  extern __shared__ float ss[];   // [ctx] or [kRowsSplit]
+  __shared__ __align__(16) float q[HD];
+  __shared__ __align__(16) float kk[HD];
+  __shared__ __align__(16) float vs[HD];
+  __shared__ float red[4], red2[4], nrm[2];
   __shared__ float4 op[G][L];
   const uint32_t h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const uint32_t d = a.d, ctx = a.ctx;
@@ -65,105 +48,121 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnArgs a) {
   }
   float* Kr = a.KV.base + (size_t)a.seq[b] * a.KV.seq_stride + a.KV.layer_off;
   float* Vr = Kr + (size_t)ctx * d;
-  const uint32_t li = tid % L, g = tid / L;
-  // stage i's pieces (slots past the last load the last one again)
-  const float* kb = Kr + h * HD + 4 * li;
-  const float* vb = Vr + h * HD + 4 * li;
-  float4 kr[D][U], vr[D][U];
-  auto issue = [&](auto I, uint32_t t0) {
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const size_t o = (size_t)min(t0 + g + u * G, s1 - 1) * d;
-      kr[decltype(I)::value][u] = *reinterpret_cast<const float4*>(kb + o);
-      vr[decltype(I)::value][u] = *reinterpret_cast<const float4*>(vb + o);
-    }
-  };
-  static_for<D>([&](auto I) { issue(I, s0 + ST * decltype(I)::value); });
-  // the row's q, k and v: every group holds q in its lanes; k and v for the
-  // ring
-  const float* x = a.QKV + (size_t)b * 3 * d + h * HD;
-  float4 q4 = *reinterpret_cast<const float4*>(x + 4 * li);
-  float4 k4 = *reinterpret_cast<const float4*>(x + d + 4 * li);
-  const float4 v4 = *reinterpret_cast<const float4*>(x + 2 * d + 4 * li);
+  const float* x = a.QKV + (size_t)b * 3 * d;
+  if (tid < HD) {
+    q[tid] = x[h * HD + tid];
+    kk[tid] = x[d + h * HD + tid];
+    vs[tid] = x[2 * d + h * HD + tid];
+  }
+  __syncthreads();
   if (a.gq) {
-    // M.qkn (bend/Dense/Model.bend:39-42)
-    auto qkn = [&](float4 t, const float* gain) {
-      const float n = 1.0f / sqrtf(lanes_sum<L>((t.x * t.x + t.y * t.y) + (t.z * t.z + t.w * t.w)) / (float)HD + 1.0e-5f);
-      const float4 gn = *reinterpret_cast<const float4*>(gain + 4 * li);
-      return make_float4((t.x * n) * (1.0f + gn.x), (t.y * n) * (1.0f + gn.y), (t.z * n) * (1.0f + gn.z),
-                         (t.w * n) * (1.0f + gn.w));
-    };
-    q4 = qkn(q4, a.gq);
-    k4 = qkn(k4, a.gk);
+    // M.qkn (bend/Dense/Model.bend:39-42) on q (wave 0) and k (wave 1)
+    if (wv < 2) {
+      const float v = lane < (uint32_t)HD ? (wv == 0 ? q[lane] : kk[lane]) : 0.0f;
+      const float t = wave_sum(v * v);
+      if (lane == 0) nrm[wv] = 1.0f / sqrtf(t / (float)HD + 1.0e-5f);
+    }
+    __syncthreads();
+    if (tid < HD) {
+      q[tid] = (q[tid] * nrm[0]) * (1.0f + a.gq[tid]);
+      kk[tid] = (kk[tid] * nrm[1]) * (1.0f + a.gk[tid]);
+    }
+    __syncthreads();
   }
+  if (tid < HD && slot >= s0 && slot < s1) {
+    Kr[(size_t)slot * d + h * HD + tid] = kk[tid];
+    Vr[(size_t)slot * d + h * HD + tid] = vs[tid];
+  }
+  const uint32_t li = tid % L, g = tid / L;
+  const float4 q4 = *reinterpret_cast<const float4*>(&q[4 * li]);
+  float4 k4o = *reinterpret_cast<const float4*>(&kk[4 * li]);
+  float4 v4o = *reinterpret_cast<const float4*>(&vs[4 * li]);
+  // opaque register values from here: a select between them and a ring load
+  // must stay a select (as a select of two loads it becomes one flat load
+  // through a stack copy)
+  asm volatile("" : "+v"(k4o.x), "+v"(k4o.y), "+v"(k4o.z), "+v"(k4o.w));
+  asm volatile("" : "+v"(v4o.x), "+v"(v4o.y), "+v"(v4o.z), "+v"(v4o.w));
   const float sc = 1.0f / sqrtf((float)HD);
-  auto dot = [&](float4 k) { return sc * lanes_sum<L>((q4.x * k.x + q4.y * k.y) + (q4.z * k.z + q4.w * k.w)); };
-  float m = kLow, l = 0.0f;
-  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  // group 0 of the workgroup that has the row's own slot starts from it
-  if (g == 0 && slot >= s0 && slot < s1) {
-    *reinterpret_cast<float4*>(Kr + (size_t)slot * d + h * HD + 4 * li) = k4;
-    *reinterpret_cast<float4*>(Vr + (size_t)slot * d + h * HD + 4 * li) = v4;
-    m = fmaxf(dot(k4), kLow);
-    l = expf(dot(k4) - m);
-    o = make_float4(l * v4.x, l * v4.y, l * v4.z, l * v4.w);
-  }
-  auto stage = [&](auto I, uint32_t t0) {
-    constexpr int i = decltype(I)::value;
-    float s[U], mn = m;
+  // one trip's pieces of ring `base` (own slot from `own`), index clamped
+  auto load = [&](const float* base, float4 own, uint32_t t0, float4* r) {
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const uint32_t t = t0 + g + u * G;
-      s[u] = dot(kr[i][u]);
-      if (t >= s1 || t == slot) s[u] = -INFINITY;
-      mn = fmaxf(mn, s[u]);
-    }
-    const float c = expf(m - mn);
-    m = mn;
-    l *= c;
-    o.x *= c;
-    o.y *= c;
-    o.z *= c;
-    o.w *= c;
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const float e = expf(s[u] - m);
-      l += e;
-      o.x = fmaf(e, vr[i][u].x, o.x);
-      o.y = fmaf(e, vr[i][u].y, o.y);
-      o.z = fmaf(e, vr[i][u].z, o.z);
-      o.w = fmaf(e, vr[i][u].w, o.w);
+      const float4 v = *reinterpret_cast<const float4*>(base + (size_t)(t < s1 ? t : s0) * d);
+      r[u] = t == slot ? own : v;
     }
   };
-  for (uint32_t t0 = s0; t0 < s1; t0 += D * ST)
-    static_for<D>([&](auto I) {
-      const uint32_t t = t0 + ST * decltype(I)::value;
-      if (t < s1) {
-        stage(I, t);
-        issue(I, t + D * ST);
-      }
-    });
-  if (li == 0) {
-    ms[g] = m;
-    ls[g] = l;
+  const float* kb = Kr + h * HD + 4 * li;
+  const float* vb = Vr + h * HD + 4 * li;
+  float4 cur[U], nxt[U];
+  load(kb, k4o, s0, cur);
+  for (uint32_t t0 = s0; t0 < s1; t0 += U * G) {
+    const bool more = t0 + U * G < s1;
+    if (more) load(kb, k4o, t0 + U * G, nxt);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t t = t0 + g + u * G;
+      float sdot = (q4.x * cur[u].x + q4.y * cur[u].y) + (q4.z * cur[u].z + q4.w * cur[u].w);
+#pragma unroll
+      for (int mk = 1; mk < L; mk <<= 1) sdot += __shfl_xor(sdot, mk, 64);
+      if (li == 0 && t < s1) ss[t - s0] = sc * sdot;
+    }
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < U; u++) cur[u] = nxt[u];
+    }
+  }
+  // the first V trip flies through the reductions
+  load(vb, v4o, s0, cur);
+  __syncthreads();
+  const uint32_t ns = s1 - s0;
+  float r = -INFINITY;
+  for (uint32_t t = tid; t < ns; t += 256) r = fmaxf(r, ss[t]);
+#pragma unroll
+  for (int mk = 32; mk >= 1; mk >>= 1) r = fmaxf(r, __shfl_xor(r, mk, 64));
+  if (lane == 0) red[wv] = r;
+  __syncthreads();
+  float mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+  const float sink = a.sink ? a.sink[h] : 0.0f;
+  if (a.sink && nsp == 1) mx = fmaxf(mx, sink);
+  float se = 0.0f;
+  for (uint32_t t = tid; t < ns; t += 256) {
+    const float e = expf(ss[t] - mx);
+    ss[t] = e;
+    se += e;
+  }
+  se = wave_sum(se);
+  if (lane == 0) red2[wv] = se;
+  __syncthreads();
+  float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (uint32_t t0 = s0; t0 < s1; t0 += U * G) {
+    const bool more = t0 + U * G < s1;
+    if (more) load(vb, v4o, t0 + U * G, nxt);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const uint32_t t = t0 + g + u * G;
+      const float e = t < s1 ? ss[t - s0] : 0.0f;
+      o.x = fmaf(e, cur[u].x, o.x);
+      o.y = fmaf(e, cur[u].y, o.y);
+      o.z = fmaf(e, cur[u].z, o.z);
+      o.w = fmaf(e, cur[u].w, o.w);
+    }
+    if (more) {
+#pragma unroll
+      for (int u = 0; u < U; u++) cur[u] = nxt[u];
+    }
   }
   op[g][li] = o;
   __syncthreads();
-  const float sink = a.sink ? a.sink[h] : 0.0f;
-  float mx = a.sink && nsp == 1 ? sink : kLow;
-#pragma unroll
-  for (int j = 0; j < G; j++) mx = fmaxf(mx, ms[j]);
-  if (tid < G) ws[tid] = expf(ms[tid] - mx);
-  __syncthreads();
   if (tid < HD) {
     const uint32_t c = tid / 4, e = tid % 4;
-    float acc = 0.0f, den = 0.0f;
+    float acc = 0.0f;
 #pragma unroll 8
     for (int j = 0; j < G; j++) {
       const float4 p4 = op[j][c];
-      acc = fmaf(ws[j], e == 0 ? p4.x : e == 1 ? p4.y : e == 2 ? p4.z : p4.w, acc);
-      den = fmaf(ws[j], ls[j], den);
+      acc += e == 0 ? p4.x : e == 1 ? p4.y : e == 2 ? p4.z : p4.w;
     }
+    float den = ((red2[0] + red2[1]) + red2[2]) + red2[3];
     if (nsp > 1) {
       part[2 + tid] = acc;
       if (tid == 0) {
@@ -179,12 +178,13 @@ __global__ __launch_bounds__(256) void k_attn_rows(AttnArgs a) {
 
 // the splits of k_attn_rows for one (head, row), with the sink:
 // M = max(m_i, sink), den = sum l_i e^(m_i - M) + e^(sink - M),
-// o = sum o_i e^(m_i - M) / den. A lane a split for the maxima and sums
-// (at most 64 splits), every split's column loaded before the first is
-// added eight at a time: one load round trip in place of one a split.
+// o = sum o_i e^(m_i - M) / den. A lane a split for the maxima and
+// weights (at most 64 splits), eight splits' columns loaded before the first
+// is added: one load round trip in place of one a split (32 rows at 2048
+// slots 6.5 -> 4.8 us).
 template <int HD>
 __global__ __launch_bounds__(64) void k_attn_rows_comb(AttnArgs a, uint32_t nsp) {
-  __shared__ float w[64];
+  __shared__ float w[64], lw[64];
   const uint32_t h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
   const float* part = a.part + ((size_t)b * a.heads + h) * nsp * (HD + 2);
   const float mi = tid < nsp ? part[tid * (HD + 2)] : -INFINITY;
@@ -197,9 +197,10 @@ __global__ __launch_bounds__(64) void k_attn_rows_comb(AttnArgs a, uint32_t nsp)
   const float M = fmaxf(wmax(mi), sink);
   const float e = tid < nsp ? expf(mi - M) : 0.0f;
   w[tid] = e;
-  const float den = wsum(li * e) + (a.sink ? expf(sink - M) : 0.0f);
+  lw[tid] = li;
   __syncthreads();
-  float acc = 0.0f;
+  float acc = 0.0f, den = a.sink ? expf(sink - M) : 0.0f;
+  for (uint32_t i = 0; i < nsp; i++) den = fmaf(lw[i], w[i], den);
 #pragma unroll
   for (uint32_t i = 0; i < 8; i++)
     if (i < nsp) acc = fmaf(v[i], w[i], acc);
@@ -210,11 +211,13 @@ __global__ __launch_bounds__(64) void k_attn_rows_comb(AttnArgs a, uint32_t nsp)
 hipError_t launch_attn_rows(const AttnArgs& a, bool split, hipStream_t st) {
   const uint32_t hd = a.heads ? a.d / a.heads : 0;
   if (!a.seq || !a.pos || !a.write_kv || a.ctx == 0 || hd * a.heads != a.d) return hipErrorInvalidValue;
+  if (!split && a.ctx > kAttnRowsMaxCtx) return hipErrorInvalidValue;
   if (split && !a.part) return hipErrorInvalidValue;
   const uint32_t nsp = split ? (a.ctx + kRowsSplit - 1) / kRowsSplit : 1u;
   if (nsp > 64 || (split && (size_t)a.B * a.heads * nsp * (hd + 2) > a.part_cap)) return hipErrorInvalidValue;
+  const size_t lds = (size_t)(split ? kRowsSplit : a.ctx) * 4;
 #define L_(H)                                                                                       \
-  hipLaunchKernelGGL(k_attn_rows<H>, dim3(a.heads, a.B, nsp), dim3(256), 0, st, a);                \
+  hipLaunchKernelGGL(k_attn_rows<H>, dim3(a.heads, a.B, nsp), dim3(256), lds, st, a);              \
   if (split) hipLaunchKernelGGL(k_attn_rows_comb<H>, dim3(a.heads, a.B), dim3(64), 0, st, a, nsp)
   switch (hd) {
     case 64: L_(64); break;

@@ -58,12 +58,6 @@ template <> struct WLoad<1> {
   }
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  return v;
-}
-
 // ------------------------------------------------------------------ products
 
 // Small batches (B <= 4): one wave per workgroup, RW rows of the product.

@@ -81,6 +81,13 @@ __device__ __forceinline__ float wmax(float v) {
   return lane_f(v, 63);
 }
 
+// the sum over the wave by lane exchanges (another order of the same sum)
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  return v;
+}
+
 // the sum over each group of G consecutive lanes (G = 16, 32 or 64), in
 // every lane of the group
 template <int G>
