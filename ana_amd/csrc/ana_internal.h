@@ -343,6 +343,12 @@ hipError_t launch_gemm_mfma(const GemvArgs& a, hipStream_t st, hipEvent_t e0 = n
                             hipEvent_t e1 = nullptr);
 // A product's weights packed for k_gemm_pk (fp32, or bf16 with bf; the
 // gains of ng folded in): pack_bytes of device memory at dst.
+// (its 16-row tiles)
+inline uint32_t pk_tiles(const GemvArgs& a) {
+  const uint32_t rows = a.mode == GM_SILU ? 2 * a.seg[0].rows
+                                          : a.seg[0].rows + (a.nseg > 1 ? a.seg[1].rows : 0);
+  return (rows + 15) / 16;
+}
 uint64_t pack_bytes(const GemvArgs& a, int bf);
 hipError_t launch_pack(const GemvArgs& a, void* dst, int bf, hipStream_t st);
 // The decode-batch GEMM over packed weights (packed with the same ng, which

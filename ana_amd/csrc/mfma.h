@@ -2,11 +2,19 @@
 // vectors, the LDS address type of global_load_lds, explicit wait counts,
 // the SiLU of the gate|up epilogues and the XCD-grouped tile order.
 #pragma once
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
 #include <type_traits>
 #include <utility>
+
+// a launch, through hipExtLaunchKernelGGL when timing events are given
+#define ANA_LAUNCH_F(K, GRID, BLOCK, LDS, ST, E0, E1, ...)                               \
+  do {                                                                                  \
+    if (E0) hipExtLaunchKernelGGL(K, GRID, BLOCK, LDS, ST, E0, E1, 0, __VA_ARGS__);      \
+    else hipLaunchKernelGGL(K, GRID, BLOCK, LDS, ST, __VA_ARGS__);                      \
+  } while (0)
 
 namespace ana {
 
