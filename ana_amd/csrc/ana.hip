@@ -755,6 +755,7 @@ static hipError_t persist_setup(ana_ctx* c) {
   if ((e = hipMemcpyAsync(c->d_play, t.data(), sizeof(PLayer) * t.size(), hipMemcpyHostToDevice, c->st)) != hipSuccess)
     return e;
   if ((e = launch_zero_u64(c->d_ll, (uint32_t)(2 * c->ll_par), c->st)) != hipSuccess) return e;
+  if ((e = launch_zero_u32(c->d_ctl, 4, c->st)) != hipSuccess) return e;
   c->pG = G;
   c->pnp = np;
   c->persist = true;
@@ -1097,6 +1098,64 @@ static int check_seqs(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* se
   return ANA_OK;
 }
 
+// what a persistent launch takes of the context (steps left 0)
+static PersistArgs persist_args(const ana_ctx* c) {
+  PersistArgs pa{};
+  pa.W = c->W;
+  pa.Wh = c->Wh;
+  pa.lay = c->d_play;
+  pa.L = c->cfg.layers; pa.d = c->cfg.d; pa.f = c->cfg.f; pa.heads = c->cfg.heads; pa.ctx = c->cfg.ctx;
+  pa.vocab = c->cfg.vocab; pa.rglru = c->cfg.rglru; pa.qk = c->cfg.qk; pa.sinks = c->cfg.sinks;
+  pa.np = c->pnp;
+  pa.exact = c->mode == ANA_EXACT_FP32 ? 1u : 0u;
+  pa.fin = c->fin;
+  pa.state = c->state; pa.seq_stride = c->seq_stride;
+  pa.X = c->X; pa.LG = c->LG;
+  pa.seq = c->d_seq; pa.pos = c->d_pos; pa.tok = c->d_tok; pa.out = c->d_out; pa.step = c->d_step;
+  pa.pick = c->d_pick;
+  pa.ll = c->d_ll; pa.ll_par = c->ll_par; pa.e_key = c->e_key;
+  pa.epoch0 = c->epoch;
+  pa.ctl = c->d_ctl;
+  pa.tmo = c->p_tmo;
+  return pa;
+}
+
+// One token into one sequence in the exact mode as one persistent launch
+// that ends before the head, its inputs by value and its residual row
+// straight into place: a step's ~60 dependent launches and copies are then
+// one, each phase's weights loaded while the
+// phase before it is exchanged; the bits are the kernels' (115M: a feed 631
+// -> 485 us; d 256, 4 layers: 174 -> 119 us). The fast modes keep the step's kernels, which
+// sum closer to the exact result than the persistent kernel does. ANA_EUNSUP,
+// having run nothing, when the launch is refused.
+static int feed_persist(ana_ctx* c, uint32_t seq, uint32_t pos, uint32_t tok) {
+  PersistArgs pa = persist_args(c);
+  pa.steps = pa.feed = 1;
+  pa.f_seq = seq; pa.f_pos = pos; pa.f_tok = tok;
+  pa.X = c->xs + (size_t)seq * c->cfg.d;
+  uint32_t ctl[4];
+  hipError_t e;
+  {
+    ProfScope ps(c, ANA_K_STEP, c->prof ? step_bytes(c, pos) - 4.0 * c->cfg.vocab * c->cfg.d : 0.0);
+    e = launch_decode1(pa, c->pG, c->st);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return ANA_EUNSUP;
+  }
+  HIPCHK(c, hipMemcpyAsync(ctl, c->d_ctl, sizeof ctl, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(c, hipStreamSynchronize(c->st));
+  c->epoch += 3;   // (no later entry carries an epoch this launch wrote)
+  if (ctl[0] || ctl[1]) {
+    // (the words stay zero between launches: only a failure raises them)
+    HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));
+    return fail(c, ANA_ETIME,
+                "persistent feed: a wait between workgroups passed its 2 s limit; the sequence's state is partly "
+                "advanced: reset it before feeding it again");
+  }
+  return ANA_OK;
+}
+
 extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint32_t* pos,
                         const uint32_t* tok) {
   if (!c) return ANA_EINVAL;
@@ -1105,6 +1164,11 @@ extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint3
   for (uint32_t i = 0; i < n; i++)
     if (tok[i] >= c->cfg.vocab) return fail(c, ANA_EINVAL, "ana_feed: token %u outside the vocabulary", tok[i]);
   HIPCHK(c, hipSetDevice(c->device));
+  if (n == 1 && !fast_mode(c) && c->persist && !c->persist_off) {
+    const int r = feed_persist(c, seq[0], pos[0], tok[0]);
+    if (r != ANA_EUNSUP) return r;
+    c->persist = false;   // refused (resources): the kernels from now on
+  }
   HIPCHK(c, hipMemcpyAsync(c->d_seq, seq, 4 * n, hipMemcpyHostToDevice, c->st));
   HIPCHK(c, hipMemcpyAsync(c->d_pos, pos, 4 * n, hipMemcpyHostToDevice, c->st));
   HIPCHK(c, hipMemcpyAsync(c->d_tok, tok, 4 * n, hipMemcpyHostToDevice, c->st));
@@ -1289,9 +1353,15 @@ extern "C" int ana_score_n(ana_ctx* c, uint32_t n, const uint32_t* seq, const ui
   return feeds_n(c, "ana_score_n", n, seq, pos, len, toks, ce);
 }
 
-static int head_of(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq) {
+// the listed sequences' residual rows, gathered (one sequence's in place)
+static int head_of(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, const float** rows) {
   if (int r = check_seqs(c, fn, n, seq)) return r;
   HIPCHK(c, hipSetDevice(c->device));
+  *rows = c->X;
+  if (n == 1) {
+    *rows = c->xs + (size_t)seq[0] * c->cfg.d;
+    return ANA_OK;
+  }
   HIPCHK(c, hipMemcpyAsync(c->d_seq, seq, 4 * n, hipMemcpyHostToDevice, c->st));
   HIPCHK(c, launch_gather_rows(c->xs, c->d_seq, n, c->cfg.d, c->X, c->st));
   return ANA_OK;
@@ -1300,8 +1370,9 @@ static int head_of(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq) 
 extern "C" int ana_logits(ana_ctx* c, uint32_t n, const uint32_t* seq, float* out) {
   if (!c) return ANA_EINVAL;
   if (!out) return fail(c, ANA_EINVAL, "ana_logits: null output");
-  if (int r = head_of(c, "ana_logits", n, seq)) return r;
-  if (int r = run_head(c, c->X, n, false)) return r;
+  const float* x;
+  if (int r = head_of(c, "ana_logits", n, seq, &x)) return r;
+  if (int r = run_head(c, x, n, false)) return r;
   HIPCHK(c, hipMemcpyAsync(out, c->LG, (size_t)4 * n * c->cfg.vocab, hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   return ANA_OK;
@@ -1311,10 +1382,11 @@ extern "C" int ana_stats(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint
                          uint32_t* alt, float* alt_prob) {
   if (!c) return ANA_EINVAL;
   if (!tok || !prob || !alt || !alt_prob) return fail(c, ANA_EINVAL, "ana_stats: null argument");
-  if (int r = head_of(c, "ana_stats", n, seq)) return r;
+  const float* x;
+  if (int r = head_of(c, "ana_stats", n, seq, &x)) return r;
   for (uint32_t i = 0; i < n; i++)
     if (tok[i] >= c->cfg.vocab) return fail(c, ANA_EINVAL, "ana_stats: token %u outside the vocabulary", tok[i]);
-  if (int r = run_head(c, c->X, n, false)) return r;
+  if (int r = run_head(c, x, n, false)) return r;
   float* dp = c->d_stat;
   float* dpa = dp + c->max_seqs;
   uint32_t* dalt = reinterpret_cast<uint32_t*>(dp + 2 * (size_t)c->max_seqs);
@@ -1330,10 +1402,11 @@ extern "C" int ana_stats(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint
 extern "C" int ana_top(ana_ctx* c, uint32_t n, const uint32_t* seq, uint32_t* tok) {
   if (!c) return ANA_EINVAL;
   if (!tok) return fail(c, ANA_EINVAL, "ana_top: null output");
-  if (int r = head_of(c, "ana_top", n, seq)) return r;
+  const float* x;
+  if (int r = head_of(c, "ana_top", n, seq, &x)) return r;
   HIPCHK(c, launch_zero_u64(c->d_amax, (uint32_t)(n * kAmaxPerRow), c->st));
-  if (int r = run_head(c, c->X, n, true)) return r;
-  if (head_keys(c, c->X, n)) HIPCHK(c, launch_keys_to_tok(c->d_amax, c->cfg.vocab, n, c->d_pick, c->st));
+  if (int r = run_head(c, x, n, true)) return r;
+  if (head_keys(c, x, n)) HIPCHK(c, launch_keys_to_tok(c->d_amax, c->cfg.vocab, n, c->d_pick, c->st));
   HIPCHK(c, hipMemcpyAsync(tok, c->d_pick, 4 * n, hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   return ANA_OK;
@@ -1359,8 +1432,9 @@ extern "C" int ana_pick(ana_ctx* c, uint32_t n, const uint32_t* seq, const ana_s
   if (!s || !tok) return fail(c, ANA_EINVAL, "ana_pick: null argument");
   const bool greedy = s->temperature <= 0.0f;
   if (!greedy && !rng) return fail(c, ANA_EINVAL, "ana_pick: sampling needs rng state");
-  if (int r = head_of(c, "ana_pick", n, seq)) return r;
-  if (int r = run_head(c, c->X, n, false)) return r;
+  const float* x;
+  if (int r = head_of(c, "ana_pick", n, seq, &x)) return r;
+  if (int r = run_head(c, x, n, false)) return r;
   if (!greedy) HIPCHK(c, hipMemcpyAsync(c->d_rng, rng, 32 * n, hipMemcpyHostToDevice, c->st));
   HIPCHK(c, launch_pick(pick_args(c, n, s, 0), c->st));
   HIPCHK(c, hipMemcpyAsync(tok, c->d_pick, 4 * n, hipMemcpyDeviceToHost, c->st));
@@ -1477,24 +1551,8 @@ static int generate_persist(ana_ctx* c, const uint32_t* pos, uint32_t steps, uin
     uint32_t done = 0;
     while (done < m) {
       HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));
-      PersistArgs pa{};
-      pa.W = c->W;
-      pa.Wh = c->Wh;
-      pa.lay = c->d_play;
-      pa.L = c->cfg.layers; pa.d = c->cfg.d; pa.f = c->cfg.f; pa.heads = c->cfg.heads; pa.ctx = c->cfg.ctx;
-      pa.vocab = c->cfg.vocab; pa.rglru = c->cfg.rglru; pa.qk = c->cfg.qk; pa.sinks = c->cfg.sinks;
-      pa.np = c->pnp;
-      pa.exact = c->mode == ANA_EXACT_FP32 ? 1u : 0u;
-      pa.fin = c->fin;
-      pa.state = c->state; pa.seq_stride = c->seq_stride;
-      pa.X = c->X; pa.LG = c->LG;
-      pa.seq = c->d_seq; pa.pos = c->d_pos; pa.tok = c->d_tok; pa.out = c->d_out; pa.step = c->d_step;
-      pa.pick = c->d_pick;
+      PersistArgs pa = persist_args(c);
       pa.steps = m - done;
-      pa.ll = c->d_ll; pa.ll_par = c->ll_par; pa.e_key = c->e_key;
-      pa.epoch0 = c->epoch;
-      pa.ctl = c->d_ctl;
-      pa.tmo = c->p_tmo;
       pa.trace = c->d_trace;
       pa.trace_steps = c->trace_steps;
       pa.trace_phases = c->trace_phases;
@@ -1517,11 +1575,13 @@ static int generate_persist(ana_ctx* c, const uint32_t* pos, uint32_t steps, uin
       HIPCHK(c, hipStreamSynchronize(c->st));
       // the next launch's entries never carry an epoch this one wrote
       c->epoch += (m - done) + 2;
-      if (ctl[0] || ctl[1])
+      if (ctl[0] || ctl[1]) {
+        HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));   // (feed_persist finds them zero)
         return fail(c, ANA_ETIME,
                     "persistent decode: a wait between workgroups passed its 2 s limit at step %u of the call; "
                     "the sequence's state is partly advanced: reset it before feeding it again",
                     k0 + done + ctl[2]);
+      }
       done += ctl[2];
       if (ctl[3]) {
         // no logit reached the maximum: Sample.argmax over the stored logits

@@ -454,6 +454,8 @@ struct PersistArgs {
   const uint32_t* seq;      // [1]
   uint32_t *pos, *tok, *out, *step, *pick;   // as ana_generate's step (out step-major)
   uint32_t steps;
+  uint32_t feed;            // one token without the head and the pick (steps 1): the states and X alone,
+  uint32_t f_seq, f_pos, f_tok;   // this one (seq, pos, tok, out and step not read or written)
   unsigned long long* ll;   // two sets of ll_par entries
   uint64_t ll_par, e_key;   // entries a set; the head's keys (one a workgroup)
   uint32_t epoch0;          // step k of the launch tags its entries epoch0 + k + 1

@@ -286,9 +286,9 @@ __global__ __launch_bounds__(kPT, 1) void k_decode1(PersistArgs a) {
   const uint32_t d = a.d, f = a.f, H = a.heads, ctx = a.ctx, L = a.L;
   if (tid == 0) bad_s = 0;
   const float* W = a.W;
-  float* Sseq = a.state + (size_t)a.seq[0] * a.seq_stride;
-  uint32_t pos = a.pos[0], tok = a.tok[0];
-  const uint32_t st0 = a.step[0];
+  float* Sseq = a.state + (size_t)(a.feed ? a.f_seq : a.seq[0]) * a.seq_stride;
+  uint32_t pos = a.feed ? a.f_pos : a.pos[0], tok = a.feed ? a.f_tok : a.tok[0];
+  const uint32_t st0 = a.feed ? 0u : a.step[0];
   const uint32_t RO = (d + G - 1) / G;          // Wo / down rows a workgroup (one a wave)
   const uint32_t RGp = (f + G - 1) / G;         // gate|up pairs a workgroup
   const uint32_t orow = w * RO + wv;            // this wave's Wo / down row
@@ -1459,6 +1459,7 @@ __global__ __launch_bounds__(kPT, 1) void k_decode1(PersistArgs a) {
       if (!ok) return;
       pb ^= 1;   // five buffer phases a layer
     }
+    if (a.feed) break;
     if (!(pb ? head(IC<1>{}, ep, LL) : head(IC<0>{}, ep, LL))) return;
     pb ^= (nhb & 1);
     bool ok = true;
@@ -1487,9 +1488,11 @@ __global__ __launch_bounds__(kPT, 1) void k_decode1(PersistArgs a) {
   __builtin_amdgcn_s_waitcnt(0);   // no load into LDS outlives the workgroup
   if (orow_ok && lane == 0) a.X[orow] = x_own;
   if (w == 0 && tid == 0) {
-    a.pos[0] = pos;
-    a.tok[0] = tok;
-    a.step[0] = st0 + k;
+    if (!a.feed) {
+      a.pos[0] = pos;
+      a.tok[0] = tok;
+      a.step[0] = st0 + k;
+    }
     if (nan_stop) a.pick[0] = v;
     a.ctl[2] = k;
     a.ctl[3] = nan_stop ? 1u : 0u;

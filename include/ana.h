@@ -93,7 +93,10 @@ int ana_config_of(const struct ana_ctx* ctx, ana_config* out, uint64_t* step);
 int ana_reset(struct ana_ctx* ctx, uint32_t seq);
 
 /* One token into each of n sequences (distinct seq[i]), no head:
- * dd.feed (bend/Dense/Decode.bend:548-551) for n sequences at once. */
+ * dd.feed (bend/Dense/Decode.bend:548-551) for n sequences at once. One
+ * sequence in ANA_EXACT_FP32 runs as one persistent launch where the device
+ * and the model allow it (as ana_generate's greedy loop, to the same bits as
+ * the step's kernels) and can then fail with ANA_ETIME. */
 int ana_feed(struct ana_ctx* ctx, uint32_t n, const uint32_t* seq, const uint32_t* pos,
              const uint32_t* tok);
 
