@@ -157,3 +157,56 @@ def test_fast_steps(tmp_path, n, plen):
     assert _rel(out[0][0], out[1][0]) < 1e-5
     for a, b in zip(out[0][1], out[1][1]):
         assert _rel(a, b) < 1e-5
+
+
+@pytest.mark.parametrize("arms", [True, False])
+@pytest.mark.parametrize("d,heads,f", [(64, 4, 192), (128, 4, 352), (256, 4, 1024)])
+def test_exact_single_feeds(oracle, tmp_path, d, heads, f, arms):
+    """One sequence's feeds (the persistent launch without its head; hd 16,
+    32, 64) from an empty slot to past the ring's wrap, between greedy loops,
+    feeds of two sequences and a reset; states, logits and picks bit for
+    bit, a sequence beside them untouched."""
+    c, path = _model(tmp_path, d, heads, arms, ctx=32, f=f)
+    m = oracle.Model(path)
+    r = np.random.RandomState(d + arms)
+    print(f"case exact single feeds d {d} arms {arms}", flush=True)
+    with ana_amd.Decoder(path, max_seqs=3) as dec:
+        st = {q: oracle.State(m) for q in (0, 1, 2)}
+        pos = {0: 0, 1: 0, 2: 0}
+
+        def feed(seqs):
+            toks = [int(r.randint(0, c.vocab)) for _ in seqs]
+            dec.feed(seqs, [pos[q] for q in seqs], toks)
+            for q, t in zip(seqs, toks):
+                st[q].feed(pos[q], t)
+                pos[q] += 1
+
+        def check(q):
+            for l in range(c.layers):
+                assert np.array_equal(bits(dec.state(q, l)), bits(st[q].layer(l))), (q, l, pos[q])
+            assert np.array_equal(bits(dec.logits([q])[0]), bits(st[q].logits())), (q, pos[q])
+            assert int(dec.top([q])[0]) == int(oracle.top(st[q].logits()))
+
+        feed([1])
+        check(1)
+        for k in range(34):                  # the ring's wrap at 32
+            feed([2])
+            if k in (0, 1, 15, 31, 32, 33):
+                check(2)
+        feed([0, 2])
+        feed([2])
+        t = int(oracle.top(st[2].logits()))
+        ids = dec.generate([2], [pos[2]], [t], 3)
+        for g in np.asarray(ids).reshape(-1):
+            st[2].feed(pos[2], t)
+            pos[2] += 1
+            t = int(oracle.top(st[2].logits()))
+            assert int(g) == t
+        feed([2])
+        check(2)
+        check(0)
+        check(1)
+        dec.reset(2)
+        st[2], pos[2] = oracle.State(m), 0
+        feed([2])
+        check(2)
