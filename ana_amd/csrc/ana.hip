@@ -469,8 +469,8 @@ extern "C" int ana_reset(ana_ctx* c, uint32_t seq) {
   if (!c) return ANA_EINVAL;
   if (seq >= c->max_seqs) return fail(c, ANA_EINVAL, "ana_reset: sequence %u outside 0..%u", seq, c->max_seqs - 1);
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, launch_zero(c->state + (uint64_t)seq * c->seq_stride, c->seq_stride, c->st));
-  HIPCHK(c, launch_zero(c->xs + (uint64_t)seq * c->cfg.d, c->cfg.d, c->st));
+  HIPCHK(c, launch_reset(c->state + (uint64_t)seq * c->seq_stride, c->seq_stride, c->xs + (uint64_t)seq * c->cfg.d,
+                         c->cfg.d, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   return ANA_OK;
 }
@@ -888,7 +888,7 @@ struct Seg {
 static int run_layers(ana_ctx* c, uint32_t B, const uint32_t* seq, const uint32_t* pos,
                       const std::vector<Seg>* segs) {
   const ana_config& cf = c->cfg;
-  const uint32_t d = cf.d, f = cf.f;
+  const uint32_t d = cf.d;
   const float* W = c->W;
   const bool chunk = segs != nullptr;
   // ANA_BF16 prefill steps whose products run on the bf16 tiles: the mixes

@@ -270,6 +270,7 @@ hipError_t launch_picks_rows(const uint32_t* sm, uint32_t n, uint32_t steps, uin
 hipError_t launch_keys_to_tok(const unsigned long long* amax, uint32_t vocab, uint32_t B,
                               uint32_t* tok, hipStream_t st);
 hipError_t launch_zero(float* p, uint64_t n, hipStream_t st);
+hipError_t launch_reset(float* state, uint64_t n, float* x, uint32_t d, hipStream_t st);
 
 // ---------------------------------------------------------------- fast modes
 // Reassociated (tree / fused multiply-add) versions of the decode step's

@@ -210,3 +210,24 @@ def test_exact_single_feeds(oracle, tmp_path, d, heads, f, arms):
         st[2], pos[2] = oracle.State(m), 0
         feed([2])
         check(2)
+
+
+@pytest.mark.parametrize("d,heads,ctx", [(64, 4, 5), (128, 4, 64), (768, 12, 2048)])
+def test_reset_clears_one_sequence(tmp_path, d, heads, ctx):
+    """k_reset (hd 16, 32, 64; states of less than a workgroup's stores and
+    more than the grid's): the sequence's states and residual row are what a
+    slot never fed has, its neighbours' are what they were, to the bit."""
+    c, path = _model(tmp_path, d, heads, True, ctx=ctx, f=2 * d)
+    print(f"case reset d {d} ctx {ctx}", flush=True)
+    with ana_amd.Decoder(path, max_seqs=4, prefill_chunk=32) as dec:
+        fresh = [dec.state(3, l) for l in range(c.layers + 1)]
+        assert not any(a.any() for a in fresh)
+        for q in (0, 1, 2):
+            dec.feeds(q, 0, np.arange(q, q + ctx // 2 + 3, dtype=np.uint32) % c.vocab)
+        before = {q: [dec.state(q, l) for l in range(c.layers + 1)] for q in (0, 2)}
+        assert all(a.any() for a in (dec.state(1, l) for l in range(c.layers + 1)))
+        dec.reset(1)
+        for l in range(c.layers + 1):
+            assert np.array_equal(bits(dec.state(1, l)), bits(fresh[l])), l
+            for q in (0, 2):
+                assert np.array_equal(bits(dec.state(q, l)), bits(before[q][l])), (q, l)
