@@ -335,12 +335,15 @@ extern "C" int ana_open(const char* path, const ana_opts* opts, ana_ctx** out) {
   c->chunk = o.prefill_chunk;
   c->wb = std::max(c->max_seqs, c->chunk);
   // a prefill's step holds up to kStepRows rows: every sequence's chunk, or
-  // longer chunks of fewer sequences (step_chunk). Past the ring's wrap the
-  // steps keep to the context's chunk, and so do the fast attention's
-  // partials, which only those steps need for more than a few rows
+  // longer chunks of fewer sequences (step_chunk; never in ANA_BF16). Past
+  // the ring's wrap the steps keep to the context's chunk, and so do the fast
+  // attention's partials, which only those steps need for more than a few
+  // rows
   const uint32_t wrap_rows =
       std::max<uint32_t>(c->wb, (uint32_t)std::min<uint64_t>((uint64_t)c->max_seqs * c->chunk, kStepRows));
-  c->rows = std::max<uint32_t>(wrap_rows, (uint32_t)std::min<uint64_t>((uint64_t)c->max_seqs * ck.cfg.ctx, kStepRows));
+  c->rows = wrap_rows;
+  if (c->mode != ANA_BF16)
+    c->rows = std::max<uint32_t>(c->rows, (uint32_t)std::min<uint64_t>((uint64_t)c->max_seqs * ck.cfg.ctx, kStepRows));
   // a step holds at most kMaxSegs chunks (each at least one row), and so
   // at most rows / kGlaSub + seg_cap sub-chunks
   c->seg_cap = std::min({c->max_seqs, c->rows, kMaxSegs});
@@ -1190,18 +1193,20 @@ extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint3
 // A step's chunk, at least the context's prefill chunk: as many tokens of
 // each of the `live` sequences as fill the step's rows, since a step of few
 // rows leaves the chip idle (one 1919-token prompt at 115M, fast_fp32: 30
-// steps of 64 rows 25.1 ms, 3.9 ms in one). From kRunSeqs
+// steps of 64 rows 25.1 ms, 3.5 ms in one). From kRunSeqs
 // sequences on the fast modes keep to kGlaRunMaxT tokens, where the GLA's
 // one workgroup a (head, chunk) fills the chip and moves a third of the
 // scan's bytes (64 us a layer at 8192 rows against 166 for the scan); fewer
 // sequences' longer chunks take the scan, whose sub-chunks run in parallel.
+// ANA_BF16 keeps the context's chunk for any number of sequences: a step's
+// rows decide which activations and weights round to bf16 (under kBigB rows
+// the first block stays in fp32), so longer steps would move its results,
+// and away from fp32 for a call of few rows; a program sets the chunk for
+// speed itself (64 prompts of 512 tokens run 1.97M tok/s at 64, 2.64M at
+// 128).
 constexpr uint32_t kRunSeqs = 16;
-// ANA_BF16 calls of kRunSeqs sequences or more keep the context's chunk: a
-// chunk's length moves where activations round to bf16, and picks near a tie
-// follow (such callers set the chunk for speed themselves: 64 prompts of 512
-// tokens run 1.97M tok/s at 64, 2.64M at 128).
-static uint32_t step_chunk(const ana_ctx* c, uint32_t n, uint32_t live) {
-  if (c->mode == ANA_BF16 && n >= kRunSeqs) return c->chunk;
+static uint32_t step_chunk(const ana_ctx* c, uint32_t live) {
+  if (c->mode == ANA_BF16) return c->chunk;
   uint32_t C = c->rows / live;
   if (fast_mode(c) && live >= kRunSeqs) C = std::min(C, kGlaRunMaxT);
   return std::max(C & ~63u, c->chunk);
@@ -1307,14 +1312,14 @@ static int feeds_n(ana_ctx* c, const char* fn, uint32_t n, const uint32_t* seq, 
       past = past || (uint64_t)pos[i] + at[i] >= c->cfg.ctx;
     }
     if (!live) break;
-    const uint32_t C = past ? c->chunk : step_chunk(c, n, live);
+    const uint32_t C = past ? c->chunk : step_chunk(c, live);
     for (uint32_t i = 0; i < n; i++) {
       const uint32_t t0 = at[i];
       if (flen[i] <= t0) continue;
       uint32_t T = std::min(C, flen[i] - t0);
-      // up to the ring's wrap in one chunk, the rest past it
+      // a chunk longer than the context's ends at the ring's wrap
       const uint64_t p0 = (uint64_t)pos[i] + t0;
-      if (p0 < c->cfg.ctx) T = (uint32_t)std::min<uint64_t>(T, c->cfg.ctx - p0);
+      if (C > c->chunk && p0 < c->cfg.ctx) T = (uint32_t)std::min<uint64_t>(T, c->cfg.ctx - p0);
       if (rows.size() + T > c->rows || segs.size() == c->seg_cap)
         if (int r = flush()) return r;
       segs.push_back(Seg{seq[i], pos[i] + t0, (uint32_t)rows.size(), T});

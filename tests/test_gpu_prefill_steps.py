@@ -159,6 +159,47 @@ def test_fast_steps(tmp_path, n, plen):
         assert _rel(a, b) < 1e-5
 
 
+@pytest.mark.parametrize("n,chunk,plen,ctx", [(1, 64, 300, 512), (3, 32, 200, 512), (15, 8, 60, 64), (2, 48, 150, 64),
+                                              (16, 64, 100, 512), (1, 128, 300, 256)])
+def test_bf16_steps_keep_the_chunk(tmp_path, n, chunk, plen, ctx):
+    """In bf16 a step's rows decide what is rounded (under 128 rows the first
+    block stays in fp32), so for any number of sequences a step is a chunk of
+    each: prompts (and scored windows) in one call are to the bit what they
+    are a chunk a call, before the ring's wrap and over it."""
+    c, path = _model(tmp_path, 256, 4, True, ctx=ctx, f=512)
+    r = np.random.RandomState(n + chunk)
+    toks = [r.randint(0, c.vocab, plen - i % 7).astype(np.uint32) for i in range(n)]
+    seqs = list(range(n))
+    print(f"case bf16 steps n {n} chunk {chunk} ctx {ctx}", flush=True)
+
+    def read(dec):
+        return [dec.logits(seqs)] + [dec.state(s, l) for s in (0, n - 1) for l in range(c.layers + 1)]
+
+    with ana_amd.Decoder(path, max_seqs=n, prefill_chunk=chunk, numerics=ana_amd.BF16) as dec:
+        dec.feeds_n(seqs, [0] * n, toks)
+        whole = read(dec)
+        for q in seqs:
+            dec.reset(q)
+        ce = dec.score_n(seqs, [0] * n, toks)
+        for q in seqs:
+            dec.reset(q)
+        for t0 in range(0, plen, chunk):
+            on = [q for q in seqs if toks[q].size > t0]
+            dec.feeds_n(on, [t0] * len(on), [toks[q][t0:t0 + chunk] for q in on])
+        parts = read(dec)
+        for q in seqs:
+            dec.reset(q)
+        pce = [[] for _ in seqs]
+        for t0 in range(0, plen - 1, chunk):
+            on = [q for q in seqs if toks[q].size - 1 > t0]
+            for q, v in zip(on, dec.score_n(on, [t0] * len(on), [toks[q][t0:t0 + chunk + 1] for q in on])):
+                pce[q].append(v)
+    for a, b in zip(whole, parts):
+        assert np.array_equal(bits(a), bits(b))
+    for a, b in zip(ce, pce):
+        assert np.array_equal(bits(a), bits(np.concatenate(b)))
+
+
 @pytest.mark.parametrize("arms", [True, False])
 @pytest.mark.parametrize("d,heads,f", [(64, 4, 192), (128, 4, 352), (256, 4, 1024)])
 def test_exact_single_feeds(oracle, tmp_path, d, heads, f, arms):
