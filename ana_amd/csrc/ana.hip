@@ -96,8 +96,8 @@ struct ana_ctx {
   };
   std::unordered_map<const float*, PkEnt> pk;
   // the persistent one-sequence decode (every mode; the exact build in ANA_EXACT_FP32): its layer table,
-  // exchange entries (two sets of ll_par), control words, grid and the
-  // epoch its next launch starts from
+  // exchange entries (two sets of ll_par), control words, grid, the epoch its
+  // next launch starts from and the tags of the head's keys
   bool persist = false, persist_off = false;
   uint32_t pG = 0, pnp = 0;
   PLayer* d_play = nullptr;
@@ -105,6 +105,7 @@ struct ana_ctx {
   uint64_t ll_par = 0, e_key = 0, ll_bytes = 0;
   uint32_t* d_ctl = nullptr;
   uint32_t epoch = 0;
+  HeadKeys hkeys;
   uint64_t p_tmo = 0;                // a wait's limit in the device clock's ticks (2 s)
   uint32_t* d_trace = nullptr;       // ana_trace's phase stamps, when armed
   uint32_t trace_steps = 0, trace_phases = 0;
@@ -1556,6 +1557,7 @@ static int generate_persist(ana_ctx* c, const uint32_t* pos, uint32_t steps, uin
     uint32_t done = 0;
     while (done < m) {
       HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));
+      c->epoch = c->hkeys.start(c->epoch);
       PersistArgs pa = persist_args(c);
       pa.steps = m - done;
       pa.trace = c->d_trace;
@@ -1582,11 +1584,16 @@ static int generate_persist(ana_ctx* c, const uint32_t* pos, uint32_t steps, uin
       c->epoch += (m - done) + 2;
       if (ctl[0] || ctl[1]) {
         HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));   // (feed_persist finds them zero)
+        // the keys of heads that not every workgroup ran
+        for (int p = 0; p < 2; p++)
+          HIPCHK(c, launch_zero_u64(c->d_ll + p * c->ll_par + c->e_key, c->pG, c->st));
+        c->hkeys.cleared();
         return fail(c, ANA_ETIME,
                     "persistent decode: a wait between workgroups passed its 2 s limit at step %u of the call; "
                     "the sequence's state is partly advanced: reset it before feeding it again",
                     k0 + done + ctl[2]);
       }
+      c->hkeys.ran(pa.epoch0, ctl);
       done += ctl[2];
       if (ctl[3]) {
         // no logit reached the maximum: Sample.argmax over the stored logits

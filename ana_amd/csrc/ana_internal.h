@@ -465,6 +465,32 @@ struct PersistArgs {
   uint32_t* trace;          // phase stamps [trace_steps][trace_phases][G][4], or null
   uint32_t trace_steps, trace_phases;
 };
+// The head's keys have 48 bits of value and index and only the low 16 bits of
+// their step's epoch, so a set's old keys must not have the tag of the next
+// head in that set. Within a launch they are those of two steps before; from
+// launch to launch the epoch may have gone round, since a launch without a
+// head (ana_feed's) moves it and leaves the keys. The host therefore keeps
+// the tags that the two sets have and starts a launch past the epochs that
+// meet them (in the kernel, tags from a count of heads took 1 to 2 us a step).
+struct HeadKeys {
+  uint32_t tag[2] = {0, 0};   // zeroed keys have tag 0
+  // the epoch0, `epoch` or a little later, from which a launch's first head in
+  // each set meets no old key
+  uint32_t start(uint32_t epoch) const {
+    while (meets(epoch + 1) || meets(epoch + 2)) epoch++;
+    return epoch;
+  }
+  // a launch from epoch0 that left control words ctl, no wait timed out, ran
+  // the heads of the steps it picked and of the one it stopped on
+  void ran(uint32_t epoch0, const uint32_t ctl[4]) {
+    const uint32_t n = ctl[2] + (ctl[3] ? 1u : 0u);
+    for (uint32_t k = n < 2 ? 0 : n - 2; k < n; k++) tag[(epoch0 + k + 1) & 1] = (epoch0 + k + 1) & 0xFFFFu;
+  }
+  void cleared() { tag[0] = tag[1] = 0; }
+
+ private:
+  bool meets(uint32_t ep) const { return tag[ep & 1] == (ep & 0xFFFFu); }
+};
 // pieces of the ring a head's attention takes (one workgroup each)
 uint32_t decode1_pieces(const ana_config& c, uint32_t G);
 // whether the persistent kernel takes this configuration on G workgroups

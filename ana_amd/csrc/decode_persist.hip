@@ -1378,6 +1378,7 @@ __global__ __launch_bounds__(kPT, 1) void k_decode1(PersistArgs a) {
       unsigned long long b2 = key_s[0];
       for (int i = 1; i < 4; i++) b2 = key_s[i] > b2 ? key_s[i] : b2;
       // (value bits, 0xFFFF - index) in 48 bits, over a 16-bit epoch tag
+      // (HeadKeys keeps old keys from meeting it)
       const uint32_t ix = 0xFFFFFFFFu - (uint32_t)(b2 & 0xFFFFFFFFull);
       const unsigned long long k48 = b2 ? ((b2 >> 32) << 16) | (0xFFFFull - ix) : 0ull;
       __hip_atomic_store(LL + a.e_key + w, (k48 << 16) | (ep & 0xFFFFu), __ATOMIC_RELAXED,

@@ -38,3 +38,17 @@ def test_launchers_reject_oversized_grids(tmp_path):
     if r.stdout.startswith("skip"):
         pytest.skip(r.stdout.strip())
     assert "0 failed" in r.stdout
+
+
+@pytest.mark.skipif(not os.path.exists(CLANG), reason="amdclang++ not found")
+def test_head_keys_never_stale(tmp_path):
+    """The persistent kernel's head keys (tests/head_keys_probe.cpp): under
+    any run of feeds and loops no set of keys carries a new head's tag before
+    that head writes it."""
+    exe = str(tmp_path / "head_keys_probe")
+    subprocess.run([CLANG, "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(LIBDIR, "csrc"), os.path.join(HERE, "head_keys_probe.cpp"), "-o", exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "0 failed" in r.stdout

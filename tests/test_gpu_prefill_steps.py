@@ -253,6 +253,32 @@ def test_exact_single_feeds(oracle, tmp_path, d, heads, f, arms):
         check(2)
 
 
+def test_exact_loops_after_many_feeds(oracle, tmp_path):
+    """Greedy loops after as many single feeds as turn a 16-bit count of
+    epochs around (three a feed): to the tag that the context's untouched
+    keys have, and from a loop's second step to the next loop's first one.
+    Picks and logits bit for bit."""
+    c, path = _model(tmp_path, 64, 4, True, ctx=32)
+    m = oracle.Model(path)
+    with ana_amd.Decoder(path, max_seqs=1) as dec:
+        for feeds in (21845, 21844):
+            print(f"case loops after {feeds} feeds", flush=True)
+            for k in range(feeds - 1):   # (and the one below)
+                dec.feed([0], [k % 40], [k % c.vocab])
+            dec.reset(0)
+            st = oracle.State(m)
+            dec.feed([0], [0], [7])
+            st.feed(0, 7)
+            t = int(oracle.top(st.logits()))
+            want = [t]
+            for k in range(5):
+                st.feed(1 + k, want[-1])
+                want.append(int(oracle.top(st.logits())))
+            got = dec.generate([0], [1], [t], 5)
+            assert np.asarray(got).reshape(-1).tolist() == want[1:], feeds
+            assert np.array_equal(bits(dec.logits([0])[0]), bits(st.logits())), feeds
+
+
 @pytest.mark.parametrize("d,heads,ctx", [(64, 4, 5), (128, 4, 64), (768, 12, 2048)])
 def test_reset_clears_one_sequence(tmp_path, d, heads, ctx):
     """k_reset (hd 16, 32, 64; states of less than a workgroup's stores and
