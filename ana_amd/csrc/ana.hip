@@ -98,7 +98,9 @@ struct ana_ctx {
   // the persistent one-sequence decode (every mode; the exact build in ANA_EXACT_FP32): its layer table,
   // exchange entries (two sets of ll_par), control words, grid, the epoch its
   // next launch starts from and the tags of the head's keys
-  bool persist = false, persist_off = false;
+  // (feed_off: a feed's launch has timed out; feed_save: the GLA states a feed replaces)
+  bool persist = false, persist_off = false, feed_off = false;
+  unsigned long long* feed_save = nullptr;
   uint32_t pG = 0, pnp = 0;
   PLayer* d_play = nullptr;
   unsigned long long* d_ll = nullptr;   // uncached (uc_take), never freed
@@ -265,7 +267,7 @@ static void release(ana_ctx* c) {
   if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
   if (c->gexec_n) (void)hipGraphExecDestroy(c->gexec_n);
   uc_give(c->device, c->d_ll, c->ll_bytes);
-  void* ps[] = {c->d_play, c->d_ctl, c->d_trace, c->W, c->Wh, c->Wp, c->d_part, c->d_gla, c->state, c->xs, c->X, c->XA, c->XN, c->QKV, c->Z, c->O, c->HH, c->LG,
+  void* ps[] = {c->d_play, c->feed_save, c->d_ctl, c->d_trace, c->W, c->Wh, c->Wp, c->d_part, c->d_gla, c->state, c->xs, c->X, c->XA, c->XN, c->QKV, c->Z, c->O, c->HH, c->LG,
                 c->d_seq, c->d_pos, c->d_tok, c->d_pick, c->d_out, c->d_step, c->d_rng, c->d_amax,
                 c->d_ss, c->d_pm, c->d_gtab, c->d_grun, c->d_atab, c->d_rseq, c->d_rpos, c->SC, c->d_tgt, c->d_ce, c->d_stat, c->d_rcp,
                 c->d_sah, c->d_hh, c->d_rsc, c->PK, c->W3, c->d_a3, c->d_h3, c->d_hpc, c->d_hpctl, c->d_oh, c->d_nxh, c->d_ssp};
@@ -692,7 +694,9 @@ static hipError_t persist_setup(ana_ctx* c) {
   int rate_khz = 0;   // the constant-rate clock the kernel's waits are timed by
   if ((e = hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, c->device)) != hipSuccess) return e;
   if (rate_khz <= 0) return hipSuccess;
-  c->p_tmo = (uint64_t)rate_khz * 2000ull;
+  // (ANA_PERSIST_MS sets the limit; with 0 every launch counts as timed out)
+  const char* ms = getenv("ANA_PERSIST_MS");
+  c->p_tmo = (uint64_t)rate_khz * (ms ? strtoull(ms, nullptr, 10) : 2000ull);
   const uint32_t d = cf.d, f = cf.f, hd = d / cf.heads, np = decode1_pieces(cf, G);
   // bf16 pieces are 16 bytes of eight values: rows start on 16 bytes when
   // d and f are multiples of 8 and the matrix does
@@ -756,6 +760,11 @@ static hipError_t persist_setup(ana_ctx* c) {
     return e;
   }
   if ((e = dalloc(&c->d_ctl, 4)) != hipSuccess) return e;
+  if (exact) {
+    const uint64_t n = (uint64_t)cf.layers * d * hd;
+    if ((e = dalloc(&c->feed_save, n)) != hipSuccess) return e;
+    if ((e = launch_zero_u64(c->feed_save, (uint32_t)n, c->st)) != hipSuccess) return e;
+  }
   if ((e = hipMemcpyAsync(c->d_play, t.data(), sizeof(PLayer) * t.size(), hipMemcpyHostToDevice, c->st)) != hipSuccess)
     return e;
   if ((e = launch_zero_u64(c->d_ll, (uint32_t)(2 * c->ll_par), c->st)) != hipSuccess) return e;
@@ -1127,15 +1136,20 @@ static PersistArgs persist_args(const ana_ctx* c) {
 // One token into one sequence in the exact mode as one persistent launch
 // that ends before the head, its inputs by value and its residual row
 // straight into place: a step's ~60 dependent launches and copies are then
-// one, each phase's weights loaded while the
-// phase before it is exchanged; the bits are the kernels' (115M: a feed 631
-// -> 485 us; d 256, 4 layers: 174 -> 119 us). The fast modes keep the step's kernels, which
-// sum closer to the exact result than the persistent kernel does. ANA_EUNSUP,
-// having run nothing, when the launch is refused.
+// one, each phase's weights loaded while the phase before it is exchanged;
+// the bits are the kernels' (115M: a feed 631 -> 485 us; d 256, 4 layers:
+// 174 -> 119 us). The fast modes keep the step's kernels, which sum closer to
+// the exact result than the persistent kernel does. ANA_EUNSUP, with the
+// sequence as it was, when the launch is refused or a wait in it passes its
+// limit: the kernels then feed the token, and those to come. A launch that
+// ends early may have written this position's k and v slots and the residual
+// row, which the kernels write again, and some of the GLA states, which are
+// put back.
 static int feed_persist(ana_ctx* c, uint32_t seq, uint32_t pos, uint32_t tok) {
   PersistArgs pa = persist_args(c);
   pa.steps = pa.feed = 1;
   pa.f_seq = seq; pa.f_pos = pos; pa.f_tok = tok;
+  pa.f_save = c->feed_save;
   pa.X = c->xs + (size_t)seq * c->cfg.d;
   uint32_t ctl[4];
   hipError_t e;
@@ -1145,17 +1159,18 @@ static int feed_persist(ana_ctx* c, uint32_t seq, uint32_t pos, uint32_t tok) {
   }
   if (e != hipSuccess) {
     (void)hipGetLastError();
+    c->persist = false;   // refused (resources): the kernels from now on
     return ANA_EUNSUP;
   }
   HIPCHK(c, hipMemcpyAsync(ctl, c->d_ctl, sizeof ctl, hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   c->epoch += 3;   // (no later entry carries an epoch this launch wrote)
-  if (ctl[0] || ctl[1]) {
+  if (ctl[0] || ctl[1] || c->p_tmo == 0) {
     // (the words stay zero between launches: only a failure raises them)
     HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));
-    return fail(c, ANA_ETIME,
-                "persistent feed: a wait between workgroups passed its 2 s limit; the sequence's state is partly "
-                "advanced: reset it before feeding it again");
+    HIPCHK(c, launch_feed_undo(pa, c->st));
+    c->feed_off = true;
+    return ANA_EUNSUP;
   }
   return ANA_OK;
 }
@@ -1168,10 +1183,9 @@ extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint3
   for (uint32_t i = 0; i < n; i++)
     if (tok[i] >= c->cfg.vocab) return fail(c, ANA_EINVAL, "ana_feed: token %u outside the vocabulary", tok[i]);
   HIPCHK(c, hipSetDevice(c->device));
-  if (n == 1 && !fast_mode(c) && c->persist && !c->persist_off) {
+  if (n == 1 && !fast_mode(c) && c->persist && !c->persist_off && !c->feed_off) {
     const int r = feed_persist(c, seq[0], pos[0], tok[0]);
     if (r != ANA_EUNSUP) return r;
-    c->persist = false;   // refused (resources): the kernels from now on
   }
   HIPCHK(c, hipMemcpyAsync(c->d_seq, seq, 4 * n, hipMemcpyHostToDevice, c->st));
   HIPCHK(c, hipMemcpyAsync(c->d_pos, pos, 4 * n, hipMemcpyHostToDevice, c->st));
@@ -1582,14 +1596,14 @@ static int generate_persist(ana_ctx* c, const uint32_t* pos, uint32_t steps, uin
       HIPCHK(c, hipStreamSynchronize(c->st));
       // the next launch's entries never carry an epoch this one wrote
       c->epoch += (m - done) + 2;
-      if (ctl[0] || ctl[1]) {
+      if (ctl[0] || ctl[1] || c->p_tmo == 0) {
         HIPCHK(c, launch_zero_u32(c->d_ctl, 4, c->st));   // (feed_persist finds them zero)
         // the keys of heads that not every workgroup ran
         for (int p = 0; p < 2; p++)
           HIPCHK(c, launch_zero_u64(c->d_ll + p * c->ll_par + c->e_key, c->pG, c->st));
         c->hkeys.cleared();
         return fail(c, ANA_ETIME,
-                    "persistent decode: a wait between workgroups passed its 2 s limit at step %u of the call; "
+                    "persistent decode: a wait between workgroups passed its time limit at step %u of the call; "
                     "the sequence's state is partly advanced: reset it before feeding it again",
                     k0 + done + ctl[2]);
       }

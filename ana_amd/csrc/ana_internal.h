@@ -457,6 +457,7 @@ struct PersistArgs {
   uint32_t steps;
   uint32_t feed;            // one token without the head and the pick (steps 1): the states and X alone,
   uint32_t f_seq, f_pos, f_tok;   // this one (seq, pos, tok, out and step not read or written)
+  unsigned long long* f_save;     // [L][d][hd]: the GLA states it replaces, as entries of its epoch
   unsigned long long* ll;   // two sets of ll_par entries
   uint64_t ll_par, e_key;   // entries a set; the head's keys (one a workgroup)
   uint32_t epoch0;          // step k of the launch tags its entries epoch0 + k + 1
@@ -496,6 +497,8 @@ uint32_t decode1_pieces(const ana_config& c, uint32_t G);
 // whether the persistent kernel takes this configuration on G workgroups
 bool decode1_fits(const ana_config& c, uint32_t G, bool exact);
 hipError_t launch_decode1(const PersistArgs& a, uint32_t G, hipStream_t st);
+// after a feed that timed out: the GLA states it replaced, back in place
+hipError_t launch_feed_undo(const PersistArgs& a, hipStream_t st);
 // phases a step of the persistent kernel takes (the trace's second extent)
 uint32_t decode1_phases(const ana_config& c);
 

@@ -31,8 +31,8 @@
 //
 // Every wait is bounded in time (the device's constant-rate clock, against a
 // limit the host passes): a workgroup that waits too long, or sees another
-// one give up, raises the abort word and leaves, and the host reports a
-// time-out (the sequence's state is then partly advanced).
+// one give up, raises the abort word and leaves. The sequence's state is then
+// partly advanced: the host reports a loop's time-out, and undoes a feed's.
 // A step whose logits have no maximum (NaN) stops the launch before its
 // pick; the host picks by Sample.argmax and launches again.
 #include <hip/hip_runtime.h>
@@ -777,7 +777,13 @@ __global__ __launch_bounds__(kPT, 1) void k_decode1(PersistArgs a) {
         }
         const float qh = qa / csqrt(1.0e-6f + s0);
         const float sn = (al * svr) + (kh * vc);
-        if (on) Sseq[P.soff + (size_t)h * HD * HD + (size_t)lane * HD + c] = sn;
+        if (on) {
+          Sseq[P.soff + (size_t)h * HD * HD + (size_t)lane * HD + c] = sn;
+          // a feed keeps what it replaces for launch_feed_undo (with the
+          // store that replaces it: 12 us less than a copy kernel before the
+          // launch, which waits for a change of queues)
+          if (a.feed) a.f_save[((size_t)l * d + 4 * w + wv) * HD + lane] = ((unsigned long long)ep << 32) | __float_as_uint(svr);
+        }
         float* pr = xs + 256 + 64 * wv;   // this wave's qh_a S'_ac (past the gathered values)
         if (on) pr[lane] = qh * sn;
         __builtin_amdgcn_wave_barrier();
@@ -1535,10 +1541,27 @@ uint32_t decode1_phases(const ana_config& c) {
   return 5 * (c.layers - sm) + 6 * sm + 2;
 }
 
+// element (row `lane`, column c = 4 w + wv over all heads) of a layer's
+// states, where the launch got as far as replacing it
+__global__ __launch_bounds__(64) void k_feed_undo(PersistArgs a) {
+  const uint32_t l = blockIdx.y, c = blockIdx.x, lane = threadIdx.x, hd = a.d / a.heads;
+  if (!a.lay[l].gla || lane >= hd) return;
+  const unsigned long long e = a.f_save[((size_t)l * a.d + c) * hd + lane];
+  if ((uint32_t)(e >> 32) != a.epoch0 + 1) return;
+  float* S = a.state + (size_t)a.f_seq * a.seq_stride + a.lay[l].soff + (size_t)(c / hd) * hd * hd;
+  S[(size_t)lane * hd + c % hd] = __uint_as_float((uint32_t)e);
+}
+
+hipError_t launch_feed_undo(const PersistArgs& a, hipStream_t st) {
+  if (!a.feed || !a.f_save || a.heads == 0 || a.d / a.heads > 64) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_feed_undo, dim3(a.d, a.L), dim3(64), 0, st, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_decode1(const PersistArgs& a, uint32_t G, hipStream_t st) {
   void* args[] = {const_cast<PersistArgs*>(&a)};
   const uint32_t hd = a.d / a.heads;
-  if (a.f > 2048) return hipErrorInvalidValue;
+  if (a.f > 2048 || (a.feed && !(a.exact && a.f_save))) return hipErrorInvalidValue;
   const bool tr = a.trace && a.trace_steps;
   if (tr && a.trace_phases > kMaxTracePhases) return hipErrorInvalidValue;
   // bf16 weights: 16-byte pieces of eight values, so rows of K = d and

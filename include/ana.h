@@ -95,8 +95,10 @@ int ana_reset(struct ana_ctx* ctx, uint32_t seq);
 /* One token into each of n sequences (distinct seq[i]), no head:
  * dd.feed (bend/Dense/Decode.bend:548-551) for n sequences at once. One
  * sequence in ANA_EXACT_FP32 runs as one persistent launch where the device
- * and the model allow it (as ana_generate's greedy loop, to the same bits as
- * the step's kernels) and can then fail with ANA_ETIME. */
+ * and the model allow it, to the same bits as the step's kernels. A launch
+ * whose waits pass their limit is undone and the token fed by the kernels,
+ * which then take the context's later feeds too: ana_feed never returns
+ * ANA_ETIME. */
 int ana_feed(struct ana_ctx* ctx, uint32_t n, const uint32_t* seq, const uint32_t* pos,
              const uint32_t* tok);
 

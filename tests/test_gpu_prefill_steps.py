@@ -253,6 +253,47 @@ def test_exact_single_feeds(oracle, tmp_path, d, heads, f, arms):
         check(2)
 
 
+@pytest.mark.parametrize("arms", [True, False])
+@pytest.mark.parametrize("d,heads,f", [(64, 4, 192), (128, 4, 352), (256, 4, 1024)])
+@pytest.mark.parametrize("plen", [20, 45])
+def test_exact_feed_after_a_timeout(oracle, tmp_path, monkeypatch, d, heads, f, arms, plen):
+    """A feed whose launch counts as timed out (a limit of 0 ms) is undone
+    and fed by the kernels (before the ring's wrap at 32 and past it), and so
+    are the ones after it; a loop's time-out is reported, and the reset
+    sequence is a fresh one. States and logits bit for bit, a sequence beside
+    it untouched."""
+    c, path = _model(tmp_path, d, heads, arms, ctx=32, f=f)
+    m = oracle.Model(path)
+    r = np.random.RandomState(d + arms + plen)
+    toks = r.randint(0, c.vocab, plen + 3).astype(np.uint32)
+    monkeypatch.setenv("ANA_PERSIST_MS", "0")
+    print(f"case exact feed after a time-out d {d} arms {arms} from {plen}", flush=True)
+    with ana_amd.Decoder(path, max_seqs=2) as dec:
+        st, beside = oracle.State(m), oracle.State(m)
+
+        def check(q, want):
+            for l in range(c.layers):
+                assert np.array_equal(bits(dec.state(q, l)), bits(want.layer(l))), (q, l)
+            assert np.array_equal(bits(dec.logits([q])[0]), bits(want.logits())), q
+
+        dec.feeds(0, 0, toks[:9])
+        beside.feeds(0, toks[:9])
+        dec.feeds(1, 0, toks[:plen])
+        st.feeds(0, toks[:plen])
+        for k in range(plen, plen + 3):
+            dec.feed([1], [k], [int(toks[k])])
+            st.feed(k, int(toks[k]))
+            check(1, st)
+        with pytest.raises(ana_amd.AnaError, match="time limit"):
+            dec.generate([1], [plen + 3], [5], 4)
+        dec.reset(1)
+        dec.feed([1], [0], [6])
+        st = oracle.State(m)
+        st.feed(0, 6)
+        check(1, st)
+        check(0, beside)
+
+
 def test_exact_loops_after_many_feeds(oracle, tmp_path):
     """Greedy loops after as many single feeds as turn a 16-bit count of
     epochs around (three a feed): to the tag that the context's untouched
