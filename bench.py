@@ -335,7 +335,7 @@ def run_agent(path: str, c, mode: str) -> dict:
 def run_prefill(path: str, c, reps: int = 5) -> dict:
     """B=64 prefill on the matrix cores: 64 prompts of 512 tokens through
     ana_feeds_n at chunk 128 (8192 rows a product), in both fast modes; the
-    median of `reps` timed passes (one pass is about 25 ms, short enough for
+    median of `reps` timed passes (one pass is 12 to 35 ms, short enough for
     clock ramps to move it by a fifth)."""
     extra = {}
     for m in ("bf16", "fast_fp32"):
@@ -356,19 +356,24 @@ def run_prefill(path: str, c, reps: int = 5) -> dict:
         # sequence and layer)
         n_sm = sum(1 for i in range(c.layers) if i % 4 == 3)
         flops = 2.0 * (c.params - c.vocab * c.d) * ntok + n_sm * 2.0 * 64 * L * L * c.d
-        peak = 2500.0 if m == "bf16" else 157.3
+        # fast_fp32: a product of two fp32 values is six bf16 products of
+        # their parts on the same matrix cores
+        peak = 2500.0 if m == "bf16" else 2500.0 / 6.0
         extra[f"prefill_b64_{m}"] = {
             "tok_s": round(ntok / dt, 1), "seconds": round(dt, 4),
             "runs_s": [round(x, 4) for x in runs],
-            "tflops": round(flops / dt / 1e12, 2), "peak_tflops": peak,
+            "tflops": round(flops / dt / 1e12, 2), "peak_tflops": round(peak, 1),
             "frac": round(flops / dt / 1e12 / peak, 4),
             "workload": "64 prompts x 512 tokens through ana_feeds_n, chunk 128; flops = 2 x "
                         "(P - v d) per token (the products) + causal attention 2 B L^2 d per "
                         "softmax layer (the GLA scan not counted)",
             "kernels": ("products k_split + k_gemm_wide / k_gemm_dl (256 x 256 and 128 x 128 MFMA tiles, "
-                        "bf16 weights x bf16 activations, both streamed straight into LDS)" if m == "bf16" else
-                        "products k_gemm_big (128 x 128 MFMA tiles, fp32 MFMA)")
-                       + ", attention k_attn_flash (fp32 MFMA), GLA k_gla_sub + k_gla_carry",
+                        "bf16 weights x bf16 activations, both streamed straight into LDS), attention "
+                        "k_attn_flash_bf (bf16 MFMA)" if m == "bf16" else
+                        "products k_split3 + k_gemm_x3 (256 x 128 and 256 x 96 tiles, operands in three bf16 "
+                        "parts, six bf16 MFMAs a term; the peak is a sixth of bf16's), attention k_attn_flash "
+                        "(fp32 MFMA)")
+                       + ", GLA k_gla_run (fp32 MFMA)",
         }
         log(f"prefill B=64 x 512 {m}: {ntok / dt:.0f} tok/s")
         # window scoring (Evaluate.bend's window.go through ana_score_n): 64
