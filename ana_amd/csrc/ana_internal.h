@@ -391,6 +391,9 @@ hipError_t launch_gemm_big(const GemvArgs& a, hipStream_t st, hipEvent_t e0 = nu
 // instead of writing its outputs; rsc when g.ng)
 bool x3_fits(const GemvArgs& g);
 uint64_t x3_bytes(uint32_t rows, uint32_t K);
+// the tile of a product of B rows and `rows` weight rows (host only): 0 .. 3
+// for 256 x 128, 256 x 96 (not with silu), 128 x 128 and 64 x 64
+int x3_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus);
 uint64_t x3_weight_bytes(const GemvArgs& g);
 hipError_t launch_pack3(const GemvArgs& g, void* dst, hipStream_t st);
 hipError_t launch_split3(const float* X, uint32_t ldx, uint32_t K, uint32_t B, void* dst, float* rsc, hipStream_t st);

@@ -318,7 +318,17 @@ struct Tile { uint32_t bm, bn, per; float round, part[3]; };
 constexpr Tile kTiles[] = {{256, 128, 1, 57.0f, {}}, {256, 96, 1, 47.0f, {}}, {128, 128, 1, 33.0f, {}},
                            {64, 64, 3, 29.0f, {0.0f, 15.0f, 20.0f}}};
 
-int pick_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus) {
+uint32_t device_cus() {
+  int dev = 0, n = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+    return 256;
+  return (uint32_t)n;
+}
+
+}  // namespace
+
+int x3_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus) {
   int best = 0;
   float least = 0.0f;
   for (int t = 0; t < 4; t++) {
@@ -333,16 +343,6 @@ int pick_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus) {
   }
   return best;
 }
-
-uint32_t device_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    return 256;
-  return (uint32_t)n;
-}
-
-}  // namespace
 
 bool x3_fits(const GemvArgs& a) {
   return a.K % 32 == 0 && a.seg[0].rows % 16 == 0 && (a.nseg < 2 || a.seg[1].rows % 16 == 0) &&
@@ -387,7 +387,7 @@ hipError_t launch_gemm_x3(const GemvArgs& g, const void* A, const void* W, const
   a.H = static_cast<__bf16*>(H);
   a.hk = silu ? g.seg[0].rows / 32 : 0;
   static const uint32_t cus = device_cus();
-  const int t = pick_tile(g.B, rows, silu, cus);
+  const int t = x3_tile(g.B, rows, silu, cus);
   const dim3 grid((rows + kTiles[t].bn - 1) / kTiles[t].bn, (g.B + kTiles[t].bm - 1) / kTiles[t].bm);
 #define L_(WM, WN, MJ, NI, S) hipLaunchKernelGGL((k_gemm_x3<WM, WN, MJ, NI, S>), grid, dim3(WM * WN * 64), 0, st, a)
   switch (t) {

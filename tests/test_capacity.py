@@ -11,6 +11,7 @@ with such arguments, on host placeholders: it runs with every device hidden
 (HIP_VISIBLE_DEVICES and ROCR_VISIBLE_DEVICES), and refuses to run a case if
 a device is still visible.
 """
+import ctypes
 import os
 import subprocess
 
@@ -52,3 +53,26 @@ def test_head_keys_never_stale(tmp_path):
     print(r.stdout)
     assert r.returncode == 0, r.stdout + r.stderr
     assert "0 failed" in r.stdout
+
+
+def test_split_tiles_covered():
+    """The cases of test_gpu_prefill_steps.test_split_products take every
+    tile of the split products (k_gemm_x3) on 256 CUs, plain and with SiLU,
+    each at least once with rows that end inside a tile."""
+    so = os.path.join(LIBDIR, "libana.so")
+    if not os.path.exists(so):
+        pytest.skip("libana.so is not built")
+    from test_gpu_prefill_steps import SPLIT_CASES, split_lens
+    tile = ctypes.CDLL(so)._ZN3ana7x3_tileEjjbj   # int ana::x3_tile(B, rows, silu, cus)
+    tile.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_bool, ctypes.c_uint32]
+    bm = [256, 256, 128, 64]
+    seen, ragged = set(), set()
+    for d, _, f, n, plen in SPLIT_CASES:
+        rows = sum(split_lens(n, plen))
+        for w, silu in ((4 * d, False), (d, False), (2 * f, True)):
+            t = tile(rows, w, silu, 256)
+            seen.add((t, silu))
+            if rows % bm[t]:
+                ragged.add((t, silu))
+    want = {(0, False), (1, False), (2, False), (3, False), (0, True), (2, True), (3, True)}
+    assert seen == want and ragged == want, (seen, ragged)

@@ -54,9 +54,17 @@ def _rel(a, b):
 
 # (d, heads, MLP, sequences, tokens of the longest): the split tiles' remainders (rows
 # past a 16-, 64- and 128-row tile, 16-row weight tiles past the last full
-# one, 2 to 64 k steps, odd numbers among them) and, at the 115M's widths, each tile shape
-@pytest.mark.parametrize("d,heads,f,n,plen", [(64, 4, 192, 2, 70), (128, 4, 160, 3, 48), (256, 4, 1024, 5, 60),
-                                              (256, 4, 352, 8, 65), (768, 12, 2048, 17, 125), (768, 12, 2048, 64, 128)])
+# one, 2 to 64 k steps, odd numbers among them) and, at the 115M's widths, each tile
+# shape, plain and SiLU (test_capacity.test_split_tiles_covered)
+SPLIT_CASES = [(64, 4, 192, 2, 70), (128, 4, 160, 3, 48), (256, 4, 1024, 5, 60), (256, 4, 352, 8, 65),
+               (768, 12, 2048, 9, 115), (768, 12, 2048, 10, 121), (768, 12, 2048, 17, 125), (768, 12, 2048, 64, 128)]
+
+
+def split_lens(n, plen):
+    return [max(1, plen - 3 * (i % 5)) for i in range(n)]
+
+
+@pytest.mark.parametrize("d,heads,f,n,plen", SPLIT_CASES)
 def test_split_products(tmp_path, d, heads, f, n, plen):
     """fast_fp32 prefill steps of 128 rows or more (k_split3, k_gemm_x3)
     against the exact mode: every state and the logits. A product's parts
@@ -64,7 +72,7 @@ def test_split_products(tmp_path, d, heads, f, n, plen):
     fp32 sums: 1e-5 is about four times what k_gemm_big's fp32 products
     show."""
     c, path = _model(tmp_path, d, heads, True, ctx=256, layers=4 if d < 768 else 2, f=f, vocab=512)
-    lens = [max(1, plen - 3 * (i % 5)) for i in range(n)]
+    lens = split_lens(n, plen)
     r = np.random.RandomState(d + f + n)
     toks = [r.randint(0, c.vocab, k).astype(np.uint32) for k in lens]
     seqs = list(range(n))
