@@ -1199,12 +1199,6 @@ extern "C" int ana_feed(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint3
   return ANA_OK;
 }
 
-// dd.feeds (bend/Dense/Decode.bend:561-639) for n sequences at once. A step
-// feeds the next chunk of every sequence that has one: their rows go through
-// each product together, the GLA and the attention chunk by chunk, so each
-// sequence ends as n separate dd.feeds would leave it (bit for bit in
-// ANA_EXACT_FP32: products are row-wise the same for any number of rows).
-
 // A step's chunk, at least the context's prefill chunk: as many tokens of
 // each of the `live` sequences as fill the step's rows, since a step of few
 // rows leaves the chip idle (one 1919-token prompt at 115M, fast_fp32: 30
@@ -1252,6 +1246,11 @@ static int score_head(ana_ctx* c, uint32_t r0, uint32_t g) {
   return ANA_OK;
 }
 
+// dd.feeds (bend/Dense/Decode.bend:561-639) for n sequences at once. A step
+// feeds the next chunk of every sequence that has one: their rows go through
+// each product together, the GLA and the attention chunk by chunk, so each
+// sequence ends as n separate dd.feeds would leave it (bit for bit in
+// ANA_EXACT_FP32: products are row-wise the same for any number of rows).
 // With ce (scoring, Evaluate.bend's window.go): sequence i feeds its first
 // len[i] - 1 tokens, and after each fed token t the head's G.lse minus the
 // logit of token t + 1 goes to ce (len[i] - 1 values a sequence, in order).
@@ -1558,8 +1557,8 @@ static int gen_inputs(ana_ctx* c, uint32_t n, const uint32_t* seq, const uint32_
   return ANA_OK;
 }
 
-// ana_generate of one greedy sequence in the fast fp32 mode: the token
-// loop as persistent launches (pieces of kOutSteps steps; a step whose
+// ana_generate of one greedy sequence, in every mode: the token loop as
+// persistent launches (pieces of kOutSteps steps; a step whose
 // logits have no maximum ends a launch, and k_advance picks it by
 // Sample.argmax before the next). Returns ANA_EUNSUP, having run nothing,
 // when the launch itself is refused (the caller then takes the graphs).

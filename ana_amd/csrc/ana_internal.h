@@ -113,6 +113,8 @@ struct Segs {
 // small-batch products take the norm and the argmax inside (B <= 4)
 constexpr uint32_t kSmallB = 4;
 // e0/e1: optional start/stop events recorded by the launch itself
+// the current device's CUs (256 when it does not say)
+uint32_t device_cus();
 hipError_t launch_gemv(const GemvArgs& a, hipStream_t st, hipEvent_t e0 = nullptr,
                        hipEvent_t e1 = nullptr);
 
@@ -429,11 +431,12 @@ hipError_t launch_zero_u32(uint32_t* p, uint32_t n, hipStream_t st);
 hipError_t launch_zero_u64(unsigned long long* p, uint32_t n, hipStream_t st);
 
 // ---------------------------------------------------------------- persistent B = 1 decode
-// The fast fp32 token loop of one sequence in one cooperative launch: one
-// workgroup a CU runs every phase of every step, phases exchanging their
-// outputs as 8-byte (value, epoch) entries. Per layer: parameter offsets
-// (floats into the parameter vector), the layer's offset in a sequence's
-// state, and its exchange slots (entries into one parity's set).
+// The greedy token loop of one sequence in one cooperative launch (every
+// mode; the exact build also feeds a single token): one workgroup a CU runs
+// every phase of every step, phases exchanging their outputs as 8-byte
+// (value, epoch) entries. Per layer: parameter offsets (floats into the
+// parameter vector), the layer's offset in a sequence's state, and its
+// exchange slots (entries into one parity's set).
 struct PLayer {
   uint64_t ra, wq, wa, lam, gq, gk, sink, wo, rf, wg, wd;
   // the bf16 matrices' device addresses, each on 16 bytes (q|k|v, z, Wo,

@@ -1,5 +1,6 @@
-// The fast-mode token loop of one sequence (ANA_FAST_FP32, B = 1) as one
-// persistent launch per ana_generate call.
+// The greedy token loop of one sequence (B = 1) as one persistent launch per
+// ana_generate call, in every mode (the exact build for ANA_EXACT_FP32), and
+// in that build ana_feed's single token, a launch without the head.
 //
 // A decode step is ~65 dependent phases (per layer: q|k|v|z, the mix, Wo,
 // gate|up, down; the head; the pick). As separate graph nodes each phase

@@ -1,4 +1,5 @@
-// The fast modes' products of 5 .. 1023 rows over packed weights (gfx950).
+// The fast modes' products over packed weights (gfx950): decode batches of
+// 5 .. 1023 rows (kPwMaxB) and prefill steps of 5 .. 127.
 #include <hip/hip_runtime.h>
 
 #include "ana_internal.h"
@@ -63,13 +64,13 @@ hipError_t launch_pack(const GemvArgs& a, void* dst, int bf, hipStream_t st) {
   return hipGetLastError();
 }
 
-// Decode batches and prefill steps of 5..127 rows in the fast modes:
+// Decode batches of 5..1023 rows and prefill steps of 5..127 in the fast modes:
 // Y[m][n] = sum_k X[m][k] W[n][k] over packed weights (the norm gains folded
 // in when `ng` is set). A workgroup owns NT 16-row weight tiles and 16 batch
 // rows (each x fragment serves the NT tiles); K = 128 NS, and its four
-// waves take a quarter of K each (NS steps of 32 k), every wave on its own. Per step a wave issues its weight pieces
-// (coalesced 1 KB loads into a ring of D register sets) and two
-// global_load_lds_dwordx4 of the 16 rows' x for that step (each 1 KB: 8 rows
+// waves take a quarter of K each (NS steps of 32 k), every wave on its own.
+// Per step a wave issues its weight pieces (coalesced 1 KB loads into a ring
+// of D register sets) and two global_load_lds_dwordx4 of the 16 rows' x for that step (each 1 KB: 8 rows
 // x 128 bytes, a row's 16-byte units at unit ^ (row & 7), so the fragment
 // reads of 16 rows at one k fall in distinct bank groups) into an LDS block
 // of its own. Its loads retire in issue order: before step s it waits until
@@ -78,9 +79,9 @@ hipError_t launch_pack(const GemvArgs& a, void* dst, int bf, hipStream_t st) {
 // l holds row l % 16 of x and of the tile at k = 8 (l / 16) + e of the step;
 // fp32 (WT 0) takes v_mfma_f32_16x16x4f32 once per e, bf16 (WT 1) one
 // v_mfma_f32_16x16x32_bf16 on x rounded to bf16. With `ng`
-// each wave also sums its rows' x^2 from the same fragments. The waves' partial tiles and sums meet in
-// LDS, where wave w adds result row r = w of every lane's four in wave order
-// and applies the norm scale 1/sqrt(ss/K + 1e-5) and the epilogue (plain,
+// each wave also sums its rows' x^2 from the same fragments. The waves'
+// partial tiles and sums meet in LDS, where wave w adds result row r = w of
+// every lane's four in wave order and applies the norm scale 1/sqrt(ss/K + 1e-5) and the epilogue (plain,
 // residual, SiLU with tile rows 0..7 gate j and 8..15 up j): with all of it
 // left to wave 0 a launch took 0.5 us more on average (B = 64, in a chain of
 // a layer's four products: fp32 8.68 -> 8.14 us a product, bf16 6.70 ->

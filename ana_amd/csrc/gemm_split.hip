@@ -318,14 +318,6 @@ struct Tile { uint32_t bm, bn, per; float round, part[3]; };
 constexpr Tile kTiles[] = {{256, 128, 1, 57.0f, {}}, {256, 96, 1, 47.0f, {}}, {128, 128, 1, 33.0f, {}},
                            {64, 64, 3, 29.0f, {0.0f, 15.0f, 20.0f}}};
 
-uint32_t device_cus() {
-  int dev = 0, n = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-    return 256;
-  return (uint32_t)n;
-}
-
 }  // namespace
 
 int x3_tile(uint32_t B, uint32_t rows, bool silu, uint32_t cus) {

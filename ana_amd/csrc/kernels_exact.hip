@@ -408,7 +408,7 @@ static const uint32_t kRmax = env_u32("ANA_GEMV_RMAX", 64);
     else hipLaunchKernelGGL(K, GRID, BLOCK, LDS, ST, __VA_ARGS__);                      \
   } while (0)
 
-static uint32_t device_cus() {
+uint32_t device_cus() {
   int dev = 0, n = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)

@@ -68,7 +68,12 @@ typedef struct {
   int device;              /* HIP device ordinal */
   int numerics;            /* ANA_EXACT_FP32, ANA_FAST_FP32 or ANA_BF16 */
   uint32_t max_seqs;       /* sequences the context keeps state for (>= 1) */
-  uint32_t prefill_chunk;  /* tokens per prefill chunk; 0 = 64, as ANA_PREFILL_CHUNK */
+  uint32_t prefill_chunk;  /* tokens of each sequence a prefill step takes; 0 = 64, as
+                              ANA_PREFILL_CHUNK. In ANA_BF16, and past the ring's wrap, exactly
+                              that; else at least that, and more where the step's rows (up to
+                              8192 over its sequences) have room: a program that wants shorter
+                              steps feeds shorter pieces. In the fast modes how a prompt's
+                              values round follows its steps, so also what is fed beside it */
 } ana_opts;
 
 /* the decoding settings of bend/Decode.bend:147-148,546-548 */
