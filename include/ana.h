@@ -176,7 +176,8 @@ void ana_rng_seeded(uint64_t seed, uint64_t rng[4]);
  * one persistent launch a call in every mode where the device and the model
  * allow it (the environment's ANA_PERSIST=0 keeps it on the step graphs);
  * its results are those of the graphs (bit for bit in ANA_EXACT_FP32), and
- * it can fail with ANA_ETIME. */
+ * it can fail with ANA_ETIME (after 2 s in one wait; ANA_PERSIST_MS in the
+ * environment sets another limit, in milliseconds). */
 int ana_generate(struct ana_ctx* ctx, uint32_t n, const uint32_t* seq, const uint32_t* pos,
                  const uint32_t* tok, uint32_t steps, const ana_sampling* s, uint64_t* rng,
                  uint32_t* out);
